@@ -1292,14 +1292,14 @@ namespace {
 // the pipelined K-row GEMM where the shapes and alignment allow it, else the
 // generic kernel. Workspace: fp8_krows_bytes(m, n, k).
 size_t fp8_krows_bytes(int64_t m, int64_t n, int64_t k) {
-  if (k % 128 != 0 || m % 16 != 0 || n % 16 != 0) return 0;
+  if (k <= 0 || m % 16 != 0 || n % 16 != 0) return 0;
   return static_cast<size_t>(fp8_gemm_krows_workspace_floats(m, n, k)) * sizeof(float);
 }
 
 int fp8_gemm_krows(const uint8_t* a, int fmt_a, const float* s_a, const uint8_t* b, int fmt_b,
                    const float* s_b, int64_t m, int64_t n, int64_t k, void* out, int out_dtype,
                    void* workspace, size_t workspace_bytes, hipStream_t st) {
-  if (k % 128 == 0 && m % 16 == 0 && n % 16 == 0 && aligned16(a) && aligned16(b)) {
+  if (k > 0 && m % 16 == 0 && n % 16 == 0 && aligned16(a) && aligned16(b)) {
     const size_t need = fp8_krows_bytes(m, n, k);
     if (need > workspace_bytes || (need > 0 && workspace == nullptr))
       return fail_invalid("fp8 K-row GEMM: workspace too small");

@@ -97,7 +97,13 @@ __device__ __forceinline__ i32x8_t load_frag_krows(const uint8_t* stage, int col
 // operand (128 x 128 tiles only), loaded by the same direct-to-LDS segments
 // and read back through transposing LDS reads (load_frag_krows). Columns
 // past the edge re-read the last 16 bytes of their row (M, N multiples of
-// 16), which only feeds outputs that are never stored.
+// 16), which only feeds outputs that are never stored. Reduction rows past
+// the end of a ragged K (a token count that is no multiple of 128) are read
+// as zeros: their lanes load from kZeroRow. At 3500 tokens the 768 x 3072
+// weight gradient took 7.7 ms in the one-output-per-thread kernel that
+// served ragged token counts before.
+__device__ const u32x4_t kZeroRow = {0, 0, 0, 0};
+
 template <int BM, int BN, int WM, int WN, int NS, int FA, int FB, bool KROWS = false>
 __device__ __forceinline__ void fp8_gemm_block(
     int bid, int nblk, const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int64_t M,
@@ -144,7 +150,7 @@ __device__ __forceinline__ void fp8_gemm_block(
   const int64_t kbeg = static_cast<int64_t>(split) * k_per_split;
   int64_t kend = kbeg + k_per_split;
   if (kend > K) kend = K;
-  const int nk = static_cast<int>((kend - kbeg) / kBK);
+  const int nk = static_cast<int>((kend - kbeg + kBK - 1) / kBK);
 
   // Per-lane DMA sources: segment j = wave + i * NW covers tile rows 8j..8j+7
   // of A (j < A_SEGS) or of B; rows past the edge re-read the last row. With
@@ -171,6 +177,20 @@ __device__ __forceinline__ void fp8_gemm_block(
       kstep[i] = 1;
     }
   }
+
+  // segment i of the slice that starts koff into this split's K range
+  const int kleft = static_cast<int>(kend - kbeg);
+  auto dma_one = [&](uint8_t* st, int64_t koff, int i) {
+    const int j = wave + i * NW;
+    if constexpr (KROWS) {
+      const int trow = (j < A_SEGS ? 8 * j : 8 * (j - A_SEGS)) + seg_row;
+      const uint8_t* p = src[i] + koff * kstep[i];
+      p = koff + trow < kleft ? p : reinterpret_cast<const uint8_t*>(&kZeroRow);
+      dma_seg(st, p, 0, j);
+    } else {
+      dma_seg(st, src[i], koff, j);
+    }
+  };
 
   f32x16_t acc[FN][FM];
 #pragma unroll
@@ -222,7 +242,7 @@ __device__ __forceinline__ void fp8_gemm_block(
     const int64_t koff = static_cast<int64_t>(s < nk ? s : nk - 1) * kBK;
     if constexpr (KROWS) {
 #pragma unroll
-      for (int i = 0; i < LPW; ++i) dma_seg(smem + s * STAGE, src[i], koff * kstep[i], wave + i * NW);
+      for (int i = 0; i < LPW; ++i) dma_one(smem + s * STAGE, koff, i);
     } else {
       dma_slice<LPW, NW>(smem + s * STAGE, src, koff, wave);
     }
@@ -251,7 +271,7 @@ __device__ __forceinline__ void fp8_gemm_block(
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int d = i * LPW / NMF; d < (i + 1) * LPW / NMF; ++d)
-        dma_seg(fill, src[d], KROWS ? refill * kstep[d] : refill, wave + d * NW);
+        dma_one(fill, refill, d);
 #pragma unroll
       for (int j = i * NFR / NMF; j < (i + 1) * NFR / NMF; ++j) frag_one(nst, 0, j, a_cur, b_cur);
       __builtin_amdgcn_sched_barrier(0);
@@ -674,7 +694,7 @@ hipError_t dispatch_fp8(const uint8_t* a, const uint8_t* b, int64_t m, int64_t n
 // tile for long reductions, as for the weight gradients of the row-major
 // form, else the two-stage tile; a forced 128 x 128 configuration is kept.
 Fp8Plan plan_fp8_krows(int64_t m, int64_t n, int64_t k) {
-  const int64_t kslices = k / kBK;
+  const int64_t kslices = ceil_div(k, kBK);
   const int forced = tune(kTuneFp8Tile);
   if (forced == 1 || forced == 6 || forced == 9) return plan_for(forced, m, n, kslices, nullptr);
   if (kslices >= 16) return split_tile_plan(m, n, kslices);
@@ -846,7 +866,7 @@ hipError_t launch_fp8_backward_pair(const uint8_t* g, const uint8_t* right_codes
                                     hipStream_t stream, bool* launched) {
   *launched = false;
   if (tune(kTuneFp8Pair) == 0) return hipSuccess;
-  if (n % kBK != 0 || m % kBK != 0 || k % 16 != 0) return hipSuccess;
+  if (n % kBK != 0 || k % 16 != 0) return hipSuccess;
   // d_left [m, k] = g [m, n] . right^T; d_right^T [n, k] = g^T . left, from
   // g [m, n] and left [m, k] as K-row operands
   Fp8Plan px = plan_fp8(m, k, n);
@@ -883,7 +903,7 @@ hipError_t launch_fp8_gemm_krows(const uint8_t* a, int fmt_a, const float* s_a, 
                                  void* out, int out_dtype, int64_t ldc, float* split_ws,
                                  int64_t split_ws_floats, hipStream_t stream) {
   if (m == 0 || n == 0) return hipSuccess;
-  if (k % kBK != 0 || m % 16 != 0 || n % 16 != 0 ||
+  if (k <= 0 || m % 16 != 0 || n % 16 != 0 ||
       split_ws_floats < fp8_gemm_krows_workspace_floats(m, n, k))
     return hipErrorInvalidValue;
   if (fmt_a == kE4M3FN && fmt_b == kE4M3FN)

@@ -226,10 +226,43 @@ def test_weight_gradient_krows_plans(cfg, right_t):
                 assert torch.equal(got, ref), (cfg, sp, m, k, n, right_t)
 
 
+@pytest.mark.parametrize("right_t", [True, False])
+@pytest.mark.parametrize("m", [1, 127, 129, 1295, 3500])
+def test_weight_gradient_krows_ragged_tokens(m, right_t):
+    """Token counts that are no multiple of 128 through the K-row kernel: one
+    token, the edges of a slice, several splits. The rows behind the last
+    token hold NaN codes and must not enter the sums."""
+
+    k, n = 208, 400
+    g = rng(4000 + m)
+    qx = _finite_codes(g, (m, k), E4M3FN)
+    qg = _finite_codes(g, (m, n), E5M2)
+    s_x, s_g = np.float32(0.0123), np.float32(3.7)
+    if right_t:
+        want = ofp8.scaled_dot_codes(np.ascontiguousarray(qg.T), s_x, E5M2, qx, s_g, E4M3FN)
+    else:
+        want = ofp8.scaled_dot_codes(np.ascontiguousarray(qx.T), s_x, E4M3FN, qg, s_g, E5M2)
+
+    def followed_by_nan(codes):
+        buf = torch.full((m + 256, codes.shape[1]), 0x7F, dtype=torch.uint8, device="cuda")
+        buf[:m] = to_dev(codes)
+        return buf[:m]
+
+    qxd, qgd = followed_by_nan(qx), followed_by_nan(qg)
+    for splits in (0, 1, 3):
+        if splits > -(-m // 128):
+            continue
+        with ops.tuning(fp8_splits=splits):
+            got = _weight_grad_krows(qxd, s_x, qgd, s_g, right_t)
+        torch.cuda.synchronize()
+        assert_bf16_close(from_dev(got), bf16_round(want), tol=FP8_TOL, min_equal=None,
+                          what=f"{m}x{k}x{n} right_t={right_t} splits={splits}")
+
+
 @pytest.mark.parametrize("m,k,n", [(200, 40, 30), (256, 24, 136), (384, 128, 100)])
 def test_weight_gradient_krows_generic_shapes(m, k, n):
-    """Shapes the pipelined K-row kernel does not take (tokens not a multiple
-    of 128, or K, N not multiples of 16) go to the generic kernel."""
+    """Shapes the pipelined K-row kernel does not take (K, N not multiples of
+    16) go to the generic kernel."""
 
     g = rng(m * 3 + k + n)
     qx = _finite_codes(g, (m, k), E4M3FN)
