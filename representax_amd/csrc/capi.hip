@@ -122,10 +122,18 @@ void plan_forward(A& a, bool fast, bool skinny, int64_t m, int64_t n, int64_t k,
     a.template take<float>(skinny_workspace_floats(m, n, k, rank));
     return;
   }
-  if (fast) return;
+  if (fast) return;  // see forward_wide_tile for the scratch it takes when there is some
   a.template take<float>(m * n);  // base product
   a.template take<float>(m * n);  // adapter product
   a.template take<float>(m * rank);
+}
+
+// The persistent wide GEMM's tile id for a forward on the MFMA path (0: the
+// fused dequantizing GEMM). It reads a bf16 copy of W_b [n, k] from the
+// workspace; a call whose workspace has no room for that copy takes the fused
+// GEMM, which needs none.
+int forward_wide_tile(int64_t m, int64_t n, int64_t k, int act) {
+  return wide_plan(m, n, k, tune(kTuneInt4Tile), act, true);
 }
 
 template <typename A>
@@ -204,12 +212,13 @@ bool knob_value_ok(int knob, int v) {
     case kTuneInt4Tile:
       return v == kTileAuto || v == kTileI4_256x128 || v == kTileI4_128x128 ||
              v == kTileI4_64x128 || v == kTileI4_256x256 || v == kTileI4_128x128s2 ||
-             v == kTileI4_128x128s3 || v == kTileI4_256x128s2 || v == kTileI4L_256x192;
+             v == kTileI4_128x128s3 || v == kTileI4_256x128s2 || v == kTileI4L_256x192 ||
+             v == kTileWide_256x256 || v == kTileWide_256x192;
     case kTuneBf16Tile:
       return v == kTileAuto || v == kTileBf_256x128 || v == kTileBf_128x128 ||
              v == kTileBf_64x128 || v == kTileBf_256x256 || v == kTileBf_128x96 ||
              v == kTileBf_256x128s3 || v == kTileT4_256x128 || v == kTileT4_128x128 ||
-             v == kTileT4_64x128;
+             v == kTileT4_64x128 || v == kTileWide_256x256 || v == kTileWide_256x192;
     case kTuneFp8Tile: return v >= 0 && v < fp8_tile_count();
     case kTuneSkinnyTile: return v >= 0 && v <= skinny_tile_count();
     case kTuneSkinny2: return v >= -1 && v <= 1;
@@ -415,8 +424,11 @@ size_t rpx_int4lora_forward_workspace(int64_t m, int64_t n, int64_t k, int64_t g
     g = group_size;
   }
   Sizer s;
-  plan_forward(s, lora_fast_shape(dtype, k, ng, g, rank), lora_skinny(dtype, m, n, k, ng, g, rank), m,
-               n, k, rank);
+  const bool fast = lora_fast_shape(dtype, k, ng, g, rank);
+  const bool skinny = lora_skinny(dtype, m, n, k, ng, g, rank);
+  plan_forward(s, fast, skinny, m, n, k, rank);
+  if (fast && !skinny && m > 0 && n > 0 && forward_wide_tile(m, n, k, kActNone) != 0)
+    s.take<uint16_t>(n * k);  // W_b
   return s.used;
 }
 
@@ -514,6 +526,17 @@ int int4lora_forward_impl(const void* x, int dtype, int64_t m, int64_t k, const 
     epi.act = act.mode;
     epi.aux = act.aux;
     epi.pre_out = act.pre_out;
+    const int wide = forward_wide_tile(m, n, k, act.mode);
+    if (wide != 0) {
+      uint16_t* wb = arena.take<uint16_t>(n * k);
+      if (!arena.overflow && wide_gemm_ok(xb, k, wb, k, m, n, k, static_cast<uint16_t*>(y), n, epi)) {
+        RPX_HIP(launch_int4_dequant(packed, scale_bits, wb, n, k, pc, ng, g, st),
+                "int4lora_forward: W_b");
+        RPX_HIP(launch_gemm_wide(wide, xb, k, wb, k, m, n, k, static_cast<uint16_t*>(y), n, epi, st),
+                "int4lora_forward: GEMM over W_b");
+        return kOk;
+      }
+    }
     RPX_HIP(launch_gemm_int4(xb, k, w, m, n, k, static_cast<uint16_t*>(y), n, epi, st),
             "int4lora_forward: fused dequant GEMM");
     return kOk;
@@ -736,7 +759,17 @@ int rpx_int4lora_forward_static(const void* x, int dtype, int64_t m, int64_t k,
                                 int64_t group_size, const uint16_t* bias_bits, const void* lora_a,
                                 const void* lora_b, int64_t rank, float scaling, void* y, void* h,
                                 void* stream) {
-  const size_t need = rpx_int4lora_forward_workspace(m, n, k, group_size, rank, dtype);
+  // the wide GEMM's W_b copy is optional: a call that it does not fit takes
+  // the fused GEMM
+  int64_t ng = 1, g = k;
+  if (group_size > 0 && group_size != k && k % group_size == 0) {
+    ng = k / group_size;
+    g = group_size;
+  }
+  Sizer sizer;
+  plan_forward(sizer, lora_fast_shape(dtype, k, ng, g, rank),
+               lora_skinny(dtype, m, n, k, ng, g, rank), m, n, k, rank);
+  const size_t need = sizer.used;
   if (need > kStaticScratchBytes)
     return fail_invalid("rpx_int4lora_forward_static: the call needs " + std::to_string(need) +
                         " bytes of scratch, more than the " +

@@ -1381,10 +1381,13 @@ hipError_t dispatch_bf16(const uint16_t* a, int64_t lda, const uint16_t* b, int6
                          const LowRankEpilogue& epi, hipStream_t stream) {
   Int4Operand none;
   int cfg = tune(kTuneBf16Tile);
+  const int wide = wide_plan(m, n, k, cfg, epi.act, false);
+  if (wide != 0 && wide_gemm_ok(a, lda, b, ldb, m, n, k, out, ldc, epi))
+    return launch_gemm_wide(wide, a, lda, b, ldb, m, n, k, out, ldc, epi, stream);
   if (cfg == kTileBf_256x256)
     return run_gemm<256, 256, 2, 2, 2, 1, kBBf16>(a, lda, b, ldb, none, m, n, k, out, ldc, epi,
                                                  stream);
-  if (cfg == kTileAuto) {
+  if (cfg == kTileAuto || cfg == kTileWide_256x256 || cfg == kTileWide_256x192) {
     // Grids of at least 256 tiles of 256 x 128 take that tile with a
     // three-stage pipeline (one workgroup of 8 waves per CU): the deeper
     // prefetch pays on long reductions (the INT4 + LoRA backward at

@@ -77,6 +77,16 @@ hipError_t launch_gemm_int4t(const uint16_t* a, int64_t lda, const Int4Operand& 
 hipError_t launch_gemm_bf16(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb,
                             int64_t m, int64_t n, int64_t k, uint16_t* out, int64_t ldc,
                             const LowRankEpilogue& epi, hipStream_t stream);
+// The same product on persistent 256-row tiles (gemm_wide.hip): the tile id
+// the planner takes for a shape and activation under a tile knob's value (0:
+// the tiles above; dequant: B is dequantized for the call), whether the operands allow it, and the launch.
+int wide_plan(int64_t m, int64_t n, int64_t k, int knob, int act, bool dequant);
+bool wide_gemm_ok(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb, int64_t m,
+                  int64_t n, int64_t k, const uint16_t* out, int64_t ldc,
+                  const LowRankEpilogue& epi);
+hipError_t launch_gemm_wide(int tile, const uint16_t* a, int64_t lda, const uint16_t* b,
+                            int64_t ldb, int64_t m, int64_t n, int64_t k, uint16_t* out,
+                            int64_t ldc, const LowRankEpilogue& epi, hipStream_t stream);
 bool gemm_fast_path_ok(int64_t k, int64_t lda, int64_t ldb_elems, const void* a, const void* b,
                        int64_t ldc, const void* out);
 

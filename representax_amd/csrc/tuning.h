@@ -54,6 +54,8 @@ enum GemmTile : int {
   kTileT4_128x128 = 15,    // packed-weight input gradient 128 x 128, one workgroup per CU
   kTileT4_64x128 = 16,     // packed-weight input gradient 64 x 128, two workgroups per CU
   kTileI4L_256x192 = 17,   // INT4 256 x 192, B dequantized once per workgroup into LDS
+  kTileWide_256x256 = 18,  // persistent 256 x 256 over bf16 B (INT4: W_b dequantized first)
+  kTileWide_256x192 = 19,  // persistent 256 x 192 over bf16 B (INT4: W_b dequantized first)
 };
 
 // Sets the dynamic-LDS limit of a kernel once per device (idempotent, so
