@@ -554,7 +554,7 @@ hipError_t run_wide_jb(const uint16_t* a, int64_t lda, const uint16_t* b, int64_
 // Estimated microseconds of both forms, fitted to graph-timed sweeps of the
 // six BERT-base and Qwen3-wide projections at 700 to 32768 rows (each tile
 // forced): the wide tiles take one round per 256 tiles, each its slices and a
-// fixed epilogue, on a launch (and the forward's dequantization); k_gemm_nt's
+// fixed epilogue, on a launch; k_gemm_nt's
 // tiles run at about 0.93 PFLOP/s less what short reductions lose. A wide
 // tile must look 5% faster (10% under an activation, whose arithmetic a lone
 // workgroup per CU does not overlap): near the line both measured within 4%
@@ -568,7 +568,9 @@ int wide_plan(int64_t m, int64_t n, int64_t k, int knob, int act, bool dequant) 
   if (knob != kTileAuto) return 0;
   const double s = static_cast<double>(k) / kBK;
   const int64_t tm = ceil_div(m, 256);
-  const double first = dequant ? 8.0 : 4.0;
+  // the forward's dequantization and what a further launch costs a caller
+  // that is not running in a graph
+  const double first = dequant ? 16.0 : 4.0;
   const double t256 = first + ceil_div(tm * ceil_div(n, 256), 256) * (1.65 * s + 6.0);
   const double t192 = first + ceil_div(tm * ceil_div(n, 192), 256) * (1.30 * s + 5.0);
   const double other =

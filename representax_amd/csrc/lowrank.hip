@@ -1,4 +1,4 @@
-// Rank-r products of the LoRA adapter and the generic any-shape kernels.
+// Rank-r products of the LoRA adapter and small elementwise kernels.
 //
 //   rank_nt: out[M, r] = bf16(sum_k op(A[m, k]) R[j, k])   (h = x A^T, dh = g_a B)
 //   rank_tn: out[P, Q] = f32(bf16(sum_m op(X[m, p]) Y[m, q]))  (dB = g_a^T h,
@@ -377,58 +377,6 @@ TiledPlan plan_tiled(int64_t m, int64_t p, int64_t q) {
   return pl;
 }
 
-// ---------------------------------------------------------------------------
-// Generic strided GEMM (any shape/dtype), fp32 accumulate and output.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ float load_elem(const void* p, int dtype, int64_t idx) {
-  if (dtype == kBF16) return bf16_to_f32(static_cast<const uint16_t*>(p)[idx]);
-  return static_cast<const float*>(p)[idx];
-}
-
-__device__ __forceinline__ float int4_elem(const Int4Operand& w, int64_t row, int64_t col) {
-  const uint32_t byte = w.packed[row * w.packed_cols + col / 2];
-  const uint32_t nib = (col & 1) ? (byte >> 4) : (byte & 0xFu);
-  const float s = bf16_to_f32(w.scales[row * w.n_groups + col / w.group]);
-  const float q = static_cast<float>(static_cast<int>(nib ^ 8u) - 8);
-  return round_bf16(q * s);
-}
-
-// B(n, k) is B[n * b_sn + k * b_sk], or, for a packed INT4 operand,
-// W_b[n, k] (int4_mode 1) or W_b[k, n] (int4_mode 2).
-__global__ void __launch_bounds__(256)
-    k_generic_gemm(const void* __restrict__ A, int a_dtype, int64_t a_sm, int64_t a_sk,
-                   const void* __restrict__ B, int b_dtype, int64_t b_sn, int64_t b_sk,
-                   Int4Operand w, int int4_mode, int64_t M, int64_t N, int64_t K,
-                   float* __restrict__ out) {
-  __shared__ float sa[16][17];
-  __shared__ float sb[16][17];
-  const int tx = threadIdx.x % 16;
-  const int ty = threadIdx.x / 16;
-  const int64_t m = static_cast<int64_t>(blockIdx.y) * 16 + ty;
-  const int64_t n = static_cast<int64_t>(blockIdx.x) * 16 + tx;
-  float acc = 0.0f;
-  for (int64_t k0 = 0; k0 < K; k0 += 16) {
-    const int64_t ka = k0 + tx;
-    sa[ty][tx] = (m < M && ka < K) ? load_elem(A, a_dtype, m * a_sm + ka * a_sk) : 0.0f;
-    const int64_t nb = static_cast<int64_t>(blockIdx.x) * 16 + ty;
-    const int64_t kb = k0 + tx;
-    float bv = 0.0f;
-    if (nb < N && kb < K) {
-      if (int4_mode != 0) {
-        bv = (int4_mode == 1) ? int4_elem(w, nb, kb) : int4_elem(w, kb, nb);
-      } else {
-        bv = load_elem(B, b_dtype, nb * b_sn + kb * b_sk);
-      }
-    }
-    sb[ty][tx] = bv;
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) acc = __builtin_fmaf(sa[ty][kk], sb[tx][kk], acc);
-    __syncthreads();
-  }
-  if (m < M && n < N) out[m * N + n] = acc;
-}
-
 __global__ void __launch_bounds__(256)
     k_round_store(const float* __restrict__ in, int64_t n, int dtype, void* __restrict__ out) {
   for (int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; e < n;
@@ -696,23 +644,6 @@ hipError_t launch_transpose_bf16(const uint16_t* in, int64_t rows, int64_t cols,
 hipError_t launch_f32_to_bf16(const float* in, uint16_t* out, int64_t n, hipStream_t stream) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_f32_to_bf16, dim3(grid1d(n)), dim3(256), 0, stream, in, out, n);
-  return hipGetLastError();
-}
-
-hipError_t launch_generic_gemm(const void* a, int a_dtype, int64_t a_sm, int64_t a_sk,
-                               const void* b, int b_dtype, int64_t b_sn, int64_t b_sk,
-                               const Int4Operand* b_int4, bool int4_transposed, int64_t m,
-                               int64_t n, int64_t k, float* out, hipStream_t stream) {
-  if (m == 0 || n == 0) return hipSuccess;
-  Int4Operand w;
-  int mode = 0;
-  if (b_int4 != nullptr) {
-    w = *b_int4;
-    mode = int4_transposed ? 2 : 1;
-  }
-  const dim3 grid(static_cast<unsigned>(ceil_div(n, 16)), static_cast<unsigned>(ceil_div(m, 16)));
-  hipLaunchKernelGGL(k_generic_gemm, grid, dim3(256), 0, stream, a, a_dtype, a_sm, a_sk, b,
-                     b_dtype, b_sn, b_sk, w, mode, m, n, k, out);
   return hipGetLastError();
 }
 

@@ -1,0 +1,83 @@
+"""The float32 matrix kernels under the INT4 + LoRA linear, elementwise
+against float64 with the bound of a float32 sum.
+
+A sum of n float32 products is within n * 2^-24 * sum |a||b| of the exact one
+whatever its order (first order in 2^-24; 2^-23 below leaves room for the
+higher ones), and each later product adds its own term. The shapes sit around
+the kernels' edges: 16 x 16 and 64 x 64 outputs, K blocks of 32 and thin steps
+of 128, odd K, group scales of 2 (one element at a time) and of 64.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from representax_amd import ops
+
+pytestmark = pytest.mark.gpu
+F64 = torch.float64
+EPS = 2.0 ** -23
+
+
+def _exact_weight(packed, scales, k):
+    p = packed.to(torch.int32)
+    q = torch.stack((p & 15, p >> 4), -1).reshape(p.shape[0], -1)[:, :k]
+    q = torch.where(q < 8, q, q - 16).float()
+    s = scales.view(torch.bfloat16).float().reshape(p.shape[0], -1)
+    return (q * s.repeat_interleave(k // s.shape[1], 1)).to(torch.bfloat16).to(F64)
+
+
+# (m, k, n, r, group)
+SHAPES = [(1, 33, 5, 1, None), (63, 64, 65, 3, 2), (65, 100, 129, 16, 4), (64, 31, 64, 17, None),
+          (200, 768, 192, 65, 64), (129, 1, 70, 1, None), (3000, 96, 48, 2, 32)]
+
+
+@pytest.mark.parametrize("m,k,n,r,group", SHAPES)
+def test_float32_linear(m, k, n, r, group):
+    g = torch.Generator(device="cuda").manual_seed(m * 7 + n)
+
+    def rnd(*s):
+        return torch.randn(s, generator=g, device="cuda")
+
+    packed, scales = ops.int4_pack(rnd(n, k), group)
+    x, a, b, gy = rnd(m, k), rnd(r, k), rnd(n, r), rnd(m, n)
+    c = 1.5
+    y, h = ops.int4lora_forward(x, packed, scales, a, b, scaling=c, group_size=group)
+    dx, d_a, d_b = ops.int4lora_backward(gy, x, packed, scales, a, b, h, scaling=c,
+                                         group_size=group)
+    w = _exact_weight(packed, scales, k)
+    xd, ad, bd, gd = (t.to(F64) for t in (x, a, b, gy))
+    hd = xd @ ad.t()
+    want = {"h": hd, "y": xd @ w.t() + c * (hd @ bd.t()),
+            "dx": gd @ w + c * (gd @ bd) @ ad, "dA": c * (gd @ bd).t() @ xd,
+            "dB": c * gd.t() @ hd}
+    xa, aa, ba, ga, wa = (t.abs() for t in (xd, ad, bd, gd, w))
+    ha = xa @ aa.t()
+    gb = ga @ ba
+    bound = {"h": k * ha, "y": (k + r + 4) * (xa @ wa.t() + c * ha @ ba.t()),
+             "dx": (n + r + 4) * (ga @ wa + c * gb @ aa), "dA": (m + n + 4) * c * gb.t() @ xa,
+             "dB": (m + k + 4) * c * ga.t() @ ha}
+    for name, got in {"h": h, "y": y, "dx": dx, "dA": d_a, "dB": d_b}.items():
+        assert got.dtype == torch.float32
+        assert ((got.to(F64) - want[name]).abs() <= EPS * bound[name]).all(), name
+
+
+def test_float32_linear_keeps_infinities_nan_and_tiny_values():
+    """Non-finite operands reach exactly the outputs their products reach, and
+    products in the subnormal range are kept (no operand is split)."""
+
+    m, k, n, r = 70, 64, 80, 2
+    packed, scales = ops.int4_pack(torch.eye(n, k, device="cuda") * 7.0)
+    x = torch.zeros((m, k), device="cuda")
+    x[3, 5], x[4, 6], x[66, 63] = float("inf"), float("nan"), 1e-38
+    zero_a, zero_b = torch.zeros((r, k), device="cuda"), torch.zeros((n, r), device="cuda")
+    w = ops.int4_dequant(packed, scales, k).float()
+    y, _ = ops.int4lora_forward(x, packed, scales, zero_a, zero_b, scaling=1.0)
+    # rows 3 and 4 are NaN wherever inf or nan meets a zero weight
+    assert torch.isnan(y[4]).all()
+    assert y[3, 5] == float("inf") or torch.isnan(y[3, 5])
+    rest = [i for i in range(m) if i not in (3, 4)]
+    assert torch.equal(y[rest], x[rest] @ w.t())
+    small, _ = ops.int4lora_forward(x[65:] * 1e-4, packed, scales, zero_a, zero_b, scaling=1.0)
+    assert torch.equal(small[1, 63], (x[66, 63] * 1e-4) * w[63, 63]) and small[1, 63] != 0
