@@ -504,8 +504,8 @@ int rpx_host_fp8_quantize(const float* host_in, int64_t n, float scale, int fmt,
  * unsupported shape). */
 size_t rpx_mnr_saved_bytes(int64_t n_queries, int64_t n_documents, int64_t dim);
 
-/* *loss (device f32) = the loss; `saved` keeps the normalised rows, norms
- * and softmax rows for the backward. */
+/* *loss (device f32) = the loss; `saved` keeps the normalised rows, norms,
+ * dot products and log-sum-exps for the backward. */
 int rpx_mnr_forward(const void* queries, const void* documents, int dtype, int64_t n_queries,
                     int64_t n_documents, int64_t dim, float scale, float* loss, void* saved,
                     size_t saved_bytes, void* stream);

@@ -56,6 +56,18 @@ def test_mnr_at_the_kernel_limits(nq, nd, dim, dtype):
     test_mnr_matches_oracle(nq, nd, dim, dtype)
 
 
+@pytest.mark.parametrize("nq,nd,dim", [(15, 16, 63), (16, 17, 64), (17, 33, 68), (65, 127, 770),
+                                       (256, 256, 768), (31, 513, 97)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_mnr_at_tile_edges(nq, nd, dim, dtype):
+    """Row tiles of 16, column chunks of 64 and summed steps of 16 (the
+    embedding width dealt to eight waves, the rows to four), each with and
+    without a remainder; widths that are no multiple of 4 take the scalar
+    loads. f32 sums of at most 770 products: the bound of the cases above."""
+
+    test_mnr_matches_oracle(nq, nd, dim, dtype)
+
+
 @pytest.mark.parametrize("q_dtype,d_dtype", [(torch.bfloat16, torch.float32),
                                              (torch.float32, torch.bfloat16)])
 def test_mnr_mixed_dtypes_cast_each_set_on_its_own(q_dtype, d_dtype):
