@@ -516,6 +516,48 @@ int rpx_mnr_backward(const float* grad_loss, const void* saved, size_t saved_byt
                      int64_t n_queries, int64_t n_documents, int64_t dim, float scale,
                      void* d_queries, void* d_documents, int dtype, void* stream);
 
+/* ---------------------------------------------------------------------------
+ * Normalisations between the linears of a layer, bf16 values with f32
+ * statistics: LayerNorm and RMSNorm over the last axis
+ * (src/representax/models/components.py:110-150), and the per-head RMSNorm of
+ * queries and keys followed by the rotary rotation
+ * (src/representax/models/qwen3_vl/text.py:30-61). Weights (and the LayerNorm's
+ * bias) are f32 or bf16; every pointer is 16-byte aligned.
+ * ------------------------------------------------------------------------- */
+#define RPX_NORM_LAYER 0
+#define RPX_NORM_RMS 1
+
+/* y = norm(t) over rows [rows, size], t = x, or bf16(x + residual) when
+ * residual is given (then `sum` receives t). LayerNorm takes its weight and
+ * bias rounded to bf16. Requires size a multiple of 8, at most 4096. */
+int rpx_norm_forward(const void* x, const void* residual, const void* weight, const void* bias,
+                     int weight_dtype, int64_t rows, int64_t size, float eps, int kind, void* sum,
+                     void* y, void* stream);
+
+/* dx = the gradient of t for the gradient dy of y, plus dsum (the gradient
+ * that reaches t by its other use) when given; t as the forward normalised it. */
+int rpx_norm_backward(const void* dy, const void* dsum, const void* t, const void* weight,
+                      int weight_dtype, int64_t rows, int64_t size, float eps, int kind, void* dx,
+                      void* stream);
+
+/* y[token, h * repeat + j] = rotate(rms_norm(x[token, h])) for j < repeat:
+ * x [tokens, heads, head_dim], y [tokens, heads * repeat, head_dim], cosines and
+ * sines f32 [sequence, head_dim], the position of a token being its index
+ * modulo `sequence`. Requires head_dim 64 or 128. */
+int rpx_head_norm_forward(const void* x, const void* weight, int weight_dtype,
+                          const void* cosines, const void* sines, int64_t tokens,
+                          int64_t sequence, int64_t heads, int64_t repeat, int64_t head_dim,
+                          float eps, void* y, void* stream);
+
+/* dx [tokens, heads, head_dim] for the gradient g of y, whose element
+ * (b, s, h, d) lies at b * stride_b + s * stride_s + h * stride_h + d
+ * (multiples of 8). */
+int rpx_head_norm_backward(const void* g, int64_t stride_b, int64_t stride_s, int64_t stride_h,
+                           const void* x, const void* weight, int weight_dtype,
+                           const void* cosines, const void* sines, int64_t tokens,
+                           int64_t sequence, int64_t heads, int64_t repeat, int64_t head_dim,
+                           float eps, void* dx, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -30,6 +30,8 @@ FP8_E5M2 = 1
 ACT_GELU = 1
 ACT_SILU_MUL = 2
 ACT_ADD = 3
+NORM_LAYER = 0
+NORM_RMS = 1
 # kernel-variant knobs (rpx_set_tuning)
 TUNE_INT4_TILE = 0
 TUNE_BF16_TILE = 1
@@ -139,6 +141,15 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "rpx_mnr_saved_bytes": (ctypes.c_size_t, [_i64, _i64, _i64]),
     "rpx_mnr_forward": (_int, [_p, _p, _int, _i64, _i64, _i64, _f32, _p, _p, ctypes.c_size_t, _p]),
     "rpx_mnr_backward": (_int, [_p, _p, ctypes.c_size_t, _i64, _i64, _i64, _f32, _p, _p, _int, _p]),
+    "rpx_norm_forward": (_int, [_p, _p, _p, _p, _int, _i64, _i64, _f32, _int, _p, _p, _p]),
+    "rpx_norm_backward": (_int, [_p, _p, _p, _p, _int, _i64, _i64, _f32, _int, _p, _p]),
+    "rpx_head_norm_forward": (
+        _int, [_p, _p, _int, _p, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p, _p]
+    ),
+    "rpx_head_norm_backward": (
+        _int,
+        [_p, _i64, _i64, _i64, _p, _p, _int, _p, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p, _p],
+    ),
 }
 
 

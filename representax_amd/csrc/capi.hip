@@ -1677,4 +1677,147 @@ int rpx_mnr_backward(const float* grad_loss, const void* saved, size_t saved_byt
   return kOk;
 }
 
+// ---------------------------------------------------------------------------
+// Normalisations between the linears
+// ---------------------------------------------------------------------------
+static bool misaligned16(std::initializer_list<const void*> pointers) {
+  for (const void* p : pointers)
+    if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return true;
+  return false;
+}
+
+static int check_norm(int weight_dtype, int64_t rows, int64_t size, int kind, const char* who) {
+  RPX_TRY(check_dtype(weight_dtype));
+  if (kind != kNormLayer && kind != kNormRms)
+    return fail_invalid(std::string(who) + ": unknown norm");
+  if (rows < 0 || rows > (int64_t{1} << 31) || size < 8 || size % 8 != 0 || size > kNormMaxSize)
+    return fail_invalid(std::string(who) +
+                        ": need 0 <= rows <= 2^31 and a size that is a multiple of 8, at most 4096");
+  return kOk;
+}
+
+int rpx_norm_forward(const void* x, const void* residual, const void* weight, const void* bias,
+                     int weight_dtype, int64_t rows, int64_t size, float eps, int kind, void* sum,
+                     void* y, void* stream) {
+  RPX_TRY(check_norm(weight_dtype, rows, size, kind, "rpx_norm_forward"));
+  if (rows == 0) return kOk;
+  if (x == nullptr || weight == nullptr || y == nullptr || (kind == kNormLayer && bias == nullptr) ||
+      (residual != nullptr && sum == nullptr))
+    return fail_invalid("rpx_norm_forward: null pointer");
+  if (misaligned16({x, residual, weight, bias, sum, y}))
+    return fail_invalid("rpx_norm_forward: pointers must be 16-byte aligned");
+  const NormArgs args{static_cast<const uint16_t*>(x),
+                      static_cast<const uint16_t*>(residual),
+                      weight,
+                      bias,
+                      weight_dtype,
+                      rows,
+                      static_cast<int>(size),
+                      eps,
+                      static_cast<uint16_t*>(sum),
+                      static_cast<uint16_t*>(y)};
+  RPX_HIP(launch_norm(args, kind, false, static_cast<hipStream_t>(stream)), "rpx_norm_forward");
+  return kOk;
+}
+
+int rpx_norm_backward(const void* dy, const void* dsum, const void* t, const void* weight,
+                      int weight_dtype, int64_t rows, int64_t size, float eps, int kind, void* dx,
+                      void* stream) {
+  RPX_TRY(check_norm(weight_dtype, rows, size, kind, "rpx_norm_backward"));
+  if (rows == 0) return kOk;
+  if (dy == nullptr || t == nullptr || weight == nullptr || dx == nullptr)
+    return fail_invalid("rpx_norm_backward: null pointer");
+  if (misaligned16({dy, dsum, t, weight, dx}))
+    return fail_invalid("rpx_norm_backward: pointers must be 16-byte aligned");
+  const NormArgs args{static_cast<const uint16_t*>(dy),
+                      static_cast<const uint16_t*>(dsum),
+                      weight,
+                      nullptr,
+                      weight_dtype,
+                      rows,
+                      static_cast<int>(size),
+                      eps,
+                      static_cast<uint16_t*>(const_cast<void*>(t)),
+                      static_cast<uint16_t*>(dx)};
+  RPX_HIP(launch_norm(args, kind, true, static_cast<hipStream_t>(stream)), "rpx_norm_backward");
+  return kOk;
+}
+
+static int check_head_norm(int weight_dtype, int64_t tokens, int64_t sequence, int64_t heads,
+                           int64_t repeat, int64_t head_dim, const char* who) {
+  RPX_TRY(check_dtype(weight_dtype));
+  if (tokens < 0 || sequence < 1 || heads < 1 || heads > 65536 || repeat < 1 || repeat > 65536 ||
+      tokens > (int64_t{1} << 31) / heads)
+    return fail_invalid(std::string(who) + ": invalid extents");
+  if (head_dim != 64 && head_dim != 128)
+    return fail_invalid(std::string(who) + ": head_dim must be 64 or 128");
+  return kOk;
+}
+
+int rpx_head_norm_forward(const void* x, const void* weight, int weight_dtype,
+                          const void* cosines, const void* sines, int64_t tokens,
+                          int64_t sequence, int64_t heads, int64_t repeat, int64_t head_dim,
+                          float eps, void* y, void* stream) {
+  RPX_TRY(check_head_norm(weight_dtype, tokens, sequence, heads, repeat, head_dim,
+                          "rpx_head_norm_forward"));
+  if (tokens == 0) return kOk;
+  if (x == nullptr || weight == nullptr || cosines == nullptr || sines == nullptr || y == nullptr)
+    return fail_invalid("rpx_head_norm_forward: null pointer");
+  if (misaligned16({x, weight, cosines, sines, y}))
+    return fail_invalid("rpx_head_norm_forward: pointers must be 16-byte aligned");
+  HeadNormArgs args{};
+  args.x = static_cast<const uint16_t*>(x);
+  args.weight = weight;
+  args.weight_dtype = weight_dtype;
+  args.cosines = static_cast<const float*>(cosines);
+  args.sines = static_cast<const float*>(sines);
+  args.tokens = tokens;
+  args.sequence = sequence;
+  args.heads = static_cast<int>(heads);
+  args.repeat = static_cast<int>(repeat);
+  args.head_dim = static_cast<int>(head_dim);
+  args.eps = eps;
+  args.out = static_cast<uint16_t*>(y);
+  RPX_HIP(launch_head_norm(args, false, static_cast<hipStream_t>(stream)),
+          "rpx_head_norm_forward");
+  return kOk;
+}
+
+int rpx_head_norm_backward(const void* g, int64_t stride_b, int64_t stride_s, int64_t stride_h,
+                           const void* x, const void* weight, int weight_dtype,
+                           const void* cosines, const void* sines, int64_t tokens,
+                           int64_t sequence, int64_t heads, int64_t repeat, int64_t head_dim,
+                           float eps, void* dx, void* stream) {
+  RPX_TRY(check_head_norm(weight_dtype, tokens, sequence, heads, repeat, head_dim,
+                          "rpx_head_norm_backward"));
+  if (tokens == 0) return kOk;
+  if (g == nullptr || x == nullptr || weight == nullptr || cosines == nullptr ||
+      sines == nullptr || dx == nullptr)
+    return fail_invalid("rpx_head_norm_backward: null pointer");
+  if (misaligned16({g, x, weight, cosines, sines, dx}) || stride_b % 8 != 0 || stride_s % 8 != 0 ||
+      stride_h % 8 != 0)
+    return fail_invalid("rpx_head_norm_backward: pointers must be 16-byte aligned, strides "
+                        "multiples of 8");
+  HeadNormArgs args{};
+  args.g = static_cast<const uint16_t*>(g);
+  args.stride_b = stride_b;
+  args.stride_s = stride_s;
+  args.stride_h = stride_h;
+  args.x = static_cast<const uint16_t*>(x);
+  args.weight = weight;
+  args.weight_dtype = weight_dtype;
+  args.cosines = static_cast<const float*>(cosines);
+  args.sines = static_cast<const float*>(sines);
+  args.tokens = tokens;
+  args.sequence = sequence;
+  args.heads = static_cast<int>(heads);
+  args.repeat = static_cast<int>(repeat);
+  args.head_dim = static_cast<int>(head_dim);
+  args.eps = eps;
+  args.out = static_cast<uint16_t*>(dx);
+  RPX_HIP(launch_head_norm(args, true, static_cast<hipStream_t>(stream)),
+          "rpx_head_norm_backward");
+  return kOk;
+}
+
 }  // extern "C"

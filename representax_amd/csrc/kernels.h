@@ -282,4 +282,40 @@ hipError_t launch_mnr_backward(const float* grad_loss, const float* saved, int64
                                int64_t dim, float scale, void* dq, void* dd, int dtype,
                                hipStream_t stream);
 
+// Row normalisations with f32 statistics, bf16 values (norm.hip).
+enum NormKind : int { kNormLayer = 0, kNormRms = 1 };
+constexpr int64_t kNormMaxSize = 4096;
+
+struct NormArgs {
+  const uint16_t* x;         // the row; backward: the gradient of y
+  const uint16_t* residual;  // added to x, or nullptr; backward: the gradient of the sum by its
+                             // other use, or nullptr
+  const void* weight;
+  const void* bias;  // LayerNorm's forward only
+  int weight_dtype;
+  int64_t rows;
+  int size;  // a multiple of 8, at most kNormMaxSize
+  float eps;
+  uint16_t* sum;  // bf16(x + residual), written when there is a residual; backward: the
+                  // normalised row, read
+  uint16_t* y;    // backward: the gradient of the row
+};
+
+struct HeadNormArgs {
+  const uint16_t* g;  // backward: the gradient of the rotated heads and its strides
+  int64_t stride_b, stride_s, stride_h;
+  const uint16_t* x;  // [tokens, heads, head_dim]
+  const void* weight;
+  int weight_dtype;
+  const float* cosines;  // [sequence, head_dim]
+  const float* sines;
+  int64_t tokens, sequence;
+  int heads, repeat, head_dim;  // head_dim 64 or 128
+  float eps;
+  uint16_t* out;
+};
+
+hipError_t launch_norm(const NormArgs& args, int kind, bool backward, hipStream_t stream);
+hipError_t launch_head_norm(const HeadNormArgs& args, bool backward, hipStream_t stream);
+
 }  // namespace rpx

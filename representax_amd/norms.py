@@ -1,0 +1,276 @@
+"""The normalisations between a layer's quantized linears, through the fused
+HIP kernels where those apply: LayerNorm and RMSNorm with float32 statistics
+(src/representax/models/components.py:110-150), the residual addition before
+them, and the per-head RMSNorm of queries and keys with the rotary rotation
+after it (src/representax/models/qwen3_vl/text.py:30-61).
+
+The kernels take bf16 device values with frozen weights; everything else
+(float32, trainable norm weights, autocast, function transforms, tracing,
+other widths and layouts) runs the torch expressions, which also define the
+values: both round to bf16 at the same places.
+"""
+
+from __future__ import annotations
+
+import torch
+import torch.nn.functional as F
+
+from . import _native as nat
+from .ops import BF16, F32, _aligned, _dtype_code, _on_device, _ptr, _stream
+
+_MAX_SIZE = 4096  # elements of a row that the kernels keep in registers
+
+
+def rms_norm(value: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """The torch expression of ``RMSNorm``."""
+
+    v = value.float()
+    v = v * torch.rsqrt(v.square().mean(-1, keepdim=True) + eps)
+    return (v * weight.float()).to(value.dtype)
+
+
+def layer_norm(value, weight, bias, eps: float) -> torch.Tensor:
+    """The torch expression of ``LayerNorm``: reduced-precision layer_norm
+    keeps float32 statistics and rounds the normalized, affine-transformed
+    value once."""
+
+    return F.layer_norm(value, value.shape[-1:], weight.to(value.dtype), bias.to(value.dtype), eps)
+
+
+def _rotate_half(value: torch.Tensor) -> torch.Tensor:
+    first, second = value.chunk(2, dim=-1)
+    return torch.cat((-second, first), dim=-1)
+
+
+def rotate(value: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
+    """The rotary rotation of ``[B, S, H, D]`` by ``[1, S, D]`` angles, in float32."""
+
+    cos, sin = cos[:, :, None], sin[:, :, None]
+    return (value.float() * cos + _rotate_half(value.float()) * sin).to(value.dtype)
+
+
+# ---------------------------------------------------------------------------
+# where the kernels apply
+# ---------------------------------------------------------------------------
+def _plain(t: torch.Tensor) -> bool:
+    """An ordinary device tensor: no subclass, no function-transform wrapper."""
+
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+
+
+def _eager() -> bool:
+    """Nothing watches or rewrites torch operations: the kernels may stand
+    for several of them."""
+
+    return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch.autograd.forward_ad._current_level >= 0
+                or torch.is_autocast_enabled("cuda"))
+
+
+def _dense(t: torch.Tensor) -> bool:
+    return t.is_contiguous() and t.data_ptr() % 16 == 0
+
+
+def _frozen(size: int, device, *weights: torch.Tensor) -> bool:
+    """Weights that the kernels take: dense float32 or bf16 rows of one
+    dtype, none of which wants a gradient."""
+
+    grad = torch.is_grad_enabled()
+    return all(_plain(w) and w.device == device and w.shape == (size,) and w.dtype in (F32, BF16)
+               and w.dtype == weights[0].dtype and _dense(w) and not (grad and w.requires_grad)
+               for w in weights)
+
+
+def _row_kernel(value: torch.Tensor, *weights: torch.Tensor) -> bool:
+    size = value.shape[-1] if value.dim() else 0
+    return (_plain(value) and value.dtype == BF16 and 8 <= size <= _MAX_SIZE and size % 8 == 0
+            and 0 < value.numel() and value.numel() // size <= 1 << 31 and _dense(value)
+            and _frozen(size, value.device, *weights) and _eager())
+
+
+def _unhooked(module: torch.nn.Module, cls: type) -> bool:
+    """Calling ``module`` is calling ``cls.forward``: no subclass, hook or
+    replaced forward would see (or miss) a fused call."""
+
+    return (type(module) is cls and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                     or module._backward_pre_hooks)
+            and not torch.nn.modules.module._has_any_global_hook())
+
+
+# ---------------------------------------------------------------------------
+# the fused calls
+# ---------------------------------------------------------------------------
+def _forward(x, residual, weight, bias, kind: int, eps: float):
+    device = _on_device(x, residual, weight, bias)
+    size = x.shape[-1]
+    y = torch.empty_like(x)
+    total = None if residual is None else torch.empty_like(x)
+    nat.call("rpx_norm_forward", _ptr(x), _ptr(residual), _ptr(weight), _ptr(bias),
+             _dtype_code(weight.dtype), x.numel() // size, size, float(eps), kind, _ptr(total),
+             _ptr(y), _stream(device))
+    return total, y
+
+
+def _expression(kind: int, value, weight, bias, eps):
+    if kind == nat.NORM_RMS:
+        return rms_norm(value, weight, eps)
+    return layer_norm(value, weight, bias, eps)
+
+
+def _gradient(ctx, dy, d_total):
+    """The gradient of the normalised row for the gradients of the norm and
+    (or None) of the row's other use."""
+
+    value, weight, bias = ctx.saved_tensors
+    if dy is None:
+        return d_total
+    if torch.is_grad_enabled():  # create_graph: the gradient is differentiated again
+        y = _expression(ctx.kind, value, weight, bias, ctx.eps)
+        dx, = torch.autograd.grad(y, value, dy, create_graph=True)
+        return dx if d_total is None else dx + d_total
+    device = _on_device(value, dy)
+    size = value.shape[-1]
+    dy, d_total = _aligned(dy), _aligned(d_total)
+    dx = torch.empty_like(value)
+    nat.call("rpx_norm_backward", _ptr(dy), _ptr(d_total), _ptr(value), _ptr(weight),
+             _dtype_code(weight.dtype), value.numel() // size, size, float(ctx.eps), ctx.kind,
+             _ptr(dx), _stream(device))
+    return dx
+
+
+class NormFn(torch.autograd.Function):
+    """A LayerNorm or RMSNorm with frozen weights."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, kind, eps):
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(x, weight, bias)
+        ctx.kind, ctx.eps = kind, eps
+        return _forward(x, None, weight, bias, kind, eps)[1]
+
+    @staticmethod
+    def backward(ctx, dy):
+        return _gradient(ctx, dy, None), None, None, None, None
+
+
+class AddNormFn(torch.autograd.Function):
+    """``t = x + residual`` and its norm, with frozen weights: ``(t, norm(t))``."""
+
+    @staticmethod
+    def forward(ctx, x, residual, weight, bias, kind, eps):
+        ctx.set_materialize_grads(False)
+        total, y = _forward(x, residual, weight, bias, kind, eps)
+        ctx.save_for_backward(total, weight, bias)
+        ctx.kind, ctx.eps = kind, eps
+        return total, y
+
+    @staticmethod
+    def backward(ctx, d_total, dy):
+        dx = _gradient(ctx, dy, d_total)
+        return dx, dx, None, None, None, None
+
+
+class HeadNormFn(torch.autograd.Function):
+    """Per-head RMSNorm with a frozen weight, the rotary rotation, and each
+    head repeated ``repeat`` times: ``[B, S, H, D] -> [B, S, H * repeat, D]``."""
+
+    @staticmethod
+    def forward(ctx, x, weight, cos, sin, eps, repeat):
+        device = _on_device(x, weight, cos, sin)
+        b, s, h, d = x.shape
+        y = torch.empty((b, s, h * repeat, d), dtype=BF16, device=device)
+        nat.call("rpx_head_norm_forward", _ptr(x), _ptr(weight), _dtype_code(weight.dtype),
+                 _ptr(cos), _ptr(sin), b * s, s, h, repeat, d, float(eps), _ptr(y),
+                 _stream(device))
+        ctx.save_for_backward(x, weight, cos, sin)
+        ctx.eps, ctx.repeat = eps, repeat
+        return y
+
+    @staticmethod
+    def backward(ctx, g):
+        x, weight, cos, sin = ctx.saved_tensors
+        if torch.is_grad_enabled():  # create_graph: the gradient is differentiated again
+            y = rotate(rms_norm(x, weight, ctx.eps), cos, sin)
+            y = y.repeat_interleave(ctx.repeat, dim=2)
+            return torch.autograd.grad(y, x, g, create_graph=True)[0], None, None, None, None, None
+        device = _on_device(x, g)
+        b, s, h, d = x.shape
+        if g.stride(3) != 1 or any(n % 8 for n in g.stride()[:3]) or g.data_ptr() % 16:
+            g = _aligned(g)
+        dx = torch.empty_like(x)
+        nat.call("rpx_head_norm_backward", _ptr(g), g.stride(0), g.stride(1), g.stride(2), _ptr(x),
+                 _ptr(weight), _dtype_code(weight.dtype), _ptr(cos), _ptr(sin), b * s, s, h,
+                 ctx.repeat, d, float(ctx.eps), _ptr(dx), _stream(device))
+        return dx, None, None, None, None, None
+
+
+class LayerNorm(torch.nn.Module):
+    """Last-axis LayerNorm with float32 statistics, output in the input dtype."""
+
+    def __init__(self, size: int, eps: float, device=None) -> None:
+        super().__init__()
+        self.weight = torch.nn.Parameter(torch.ones(size, device=device))
+        self.bias = torch.nn.Parameter(torch.zeros(size, device=device))
+        self.eps = eps
+
+    def forward(self, value: torch.Tensor) -> torch.Tensor:
+        if _row_kernel(value, self.weight, self.bias):
+            return NormFn.apply(value, self.weight, self.bias, nat.NORM_LAYER, self.eps)
+        return layer_norm(value, self.weight, self.bias, self.eps)
+
+
+class RMSNorm(torch.nn.Module):
+    """Last-axis RMS normalisation with float32 statistics
+    (src/representax/models/components.py:134-150)."""
+
+    def __init__(self, size: int, eps: float, device=None) -> None:
+        super().__init__()
+        self.weight = torch.nn.Parameter(torch.ones(size, device=device))
+        self.eps = eps
+
+    def forward(self, value: torch.Tensor) -> torch.Tensor:
+        if _row_kernel(value, self.weight):
+            return NormFn.apply(value, self.weight, None, nat.NORM_RMS, self.eps)
+        return rms_norm(value, self.weight, self.eps)
+
+
+def add_norm(norm: torch.nn.Module, value: torch.Tensor, update: torch.Tensor):
+    """``t = value + update`` and ``norm(t)``: ``(t, norm(t))``, in one pass
+    where the kernels apply."""
+
+    kind = {LayerNorm: nat.NORM_LAYER, RMSNorm: nat.NORM_RMS}.get(type(norm))
+    if kind is not None and _unhooked(norm, type(norm)):
+        bias = norm.bias if kind == nat.NORM_LAYER else None
+        weights = (norm.weight,) if bias is None else (norm.weight, bias)
+        if (_row_kernel(value, *weights) and _plain(update) and update.dtype == BF16
+                and update.shape == value.shape and update.device == value.device
+                and _dense(update)):
+            return AddNormFn.apply(value, update, norm.weight, bias, kind, norm.eps)
+    total = value + update
+    return total, norm(total)
+
+
+def head_norm_rotary(norm: torch.nn.Module, heads: torch.Tensor, cos: torch.Tensor,
+                     sin: torch.Tensor, dtype: torch.dtype, repeat: int = 1) -> torch.Tensor:
+    """``norm`` of each head of ``[B, S, H, D]``, rotated by ``[1, S, D]``
+    float32 angles and rounded to ``dtype``, every head repeated ``repeat``
+    times; in one pass where the kernels apply."""
+
+    b, s, h, d = heads.shape
+    if (_unhooked(norm, RMSNorm) and d in (64, 128) and dtype == BF16
+            and _row_kernel(heads, norm.weight)
+            and all(_plain(t) and t.dtype == F32 and t.device == heads.device
+                    and t.shape == (1, s, d) and _dense(t) and not t.requires_grad
+                    for t in (cos, sin))
+            and h <= 65536 and repeat <= 65536):
+        return HeadNormFn.apply(heads, norm.weight, cos, sin, norm.eps, repeat)
+    value = norm(heads)
+    cos, sin = cos[:, :, None], sin[:, :, None]
+    value = (value.float() * cos + _rotate_half(value.float()) * sin).to(dtype)
+    return value if repeat == 1 else value.repeat_interleave(repeat, dim=2)
+
+
+__all__ = ["LayerNorm", "RMSNorm", "add_norm", "head_norm_rotary"]

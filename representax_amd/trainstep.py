@@ -44,6 +44,7 @@ from .adapters import apply_quantized_lora, lora_parameters
 from .components import Linear
 from .config import PrecisionConfig
 from .mlp import gelu_mlp, shared_input_projections, swiglu_mlp
+from .norms import LayerNorm, RMSNorm, add_norm, head_norm_rotary
 from .precision import (active_compute_views, active_policy, compute_views, precision_context,
                         resolve_precision_policy)
 
@@ -79,22 +80,6 @@ class BertConfig:
         # backward: dX through every linear and both attention products twice
         backward = self.num_hidden_layers * (linear + 2 * attention)
         return forward * (2 if remat else 1) + backward
-
-
-class LayerNorm(torch.nn.Module):
-    """Last-axis LayerNorm with float32 statistics, output in the input dtype."""
-
-    def __init__(self, size: int, eps: float, device=None) -> None:
-        super().__init__()
-        self.weight = torch.nn.Parameter(torch.ones(size, device=device))
-        self.bias = torch.nn.Parameter(torch.zeros(size, device=device))
-        self.eps = eps
-
-    def forward(self, value: torch.Tensor) -> torch.Tensor:
-        # torch's reduced-precision layer_norm keeps float32 statistics and
-        # rounds the normalized, affine-transformed value once
-        return F.layer_norm(value, value.shape[-1:], self.weight.to(value.dtype),
-                            self.bias.to(value.dtype), self.eps)
 
 
 REMAT_POLICIES = ("none", "full")
@@ -213,8 +198,8 @@ class BertLayer(torch.nn.Module):
         self.output_norm = LayerNorm(config.hidden_size, config.norm_epsilon, device)
 
     def forward(self, hidden: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
-        hidden = self.attention_norm(hidden + self.attention(hidden, bias))
-        return self.output_norm(hidden + self.mlp(hidden))
+        _, hidden = add_norm(self.attention_norm, hidden, self.attention(hidden, bias))
+        return add_norm(self.output_norm, hidden, self.mlp(hidden))[1]
 
 
 class BertEncoder(torch.nn.Module):
@@ -330,26 +315,6 @@ class Qwen3TextConfig:
         return forward * (2 if remat else 1) + backward
 
 
-class RMSNorm(torch.nn.Module):
-    """Last-axis RMS normalisation with float32 statistics
-    (src/representax/models/components.py:134-150)."""
-
-    def __init__(self, size: int, eps: float, device=None) -> None:
-        super().__init__()
-        self.weight = torch.nn.Parameter(torch.ones(size, device=device))
-        self.eps = eps
-
-    def forward(self, value: torch.Tensor) -> torch.Tensor:
-        v = value.float()
-        v = v * torch.rsqrt(v.square().mean(-1, keepdim=True) + self.eps)
-        return (v * self.weight.float()).to(value.dtype)
-
-
-def _rotate_half(value: torch.Tensor) -> torch.Tensor:
-    first, second = value.chunk(2, dim=-1)
-    return torch.cat((-second, first), dim=-1)
-
-
 class Qwen3Attention(torch.nn.Module):
     def __init__(self, config: Qwen3TextConfig, key: int, device=None) -> None:
         super().__init__()
@@ -367,16 +332,13 @@ class Qwen3Attention(torch.nn.Module):
     def forward(self, hidden, cos, sin):
         b, s, _ = hidden.shape
         q, k, v = shared_input_projections(hidden, (self.query, self.key, self.value))
-        q = self.query_norm(q.reshape(b, s, self.heads, self.head_dim))
-        k = self.key_norm(k.reshape(b, s, self.kv_heads, self.head_dim))
-        v = v.reshape(b, s, self.kv_heads, self.head_dim)
-        cos, sin = cos[:, :, None], sin[:, :, None]
-        q = (q.float() * cos + _rotate_half(q.float()) * sin).to(hidden.dtype)
-        k = (k.float() * cos + _rotate_half(k.float()) * sin).to(hidden.dtype)
         rep = self.heads // self.kv_heads
-        q, k, v = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)
+        q = head_norm_rotary(self.query_norm, q.reshape(b, s, self.heads, self.head_dim), cos, sin,
+                             hidden.dtype).transpose(1, 2)
+        k = head_norm_rotary(self.key_norm, k.reshape(b, s, self.kv_heads, self.head_dim), cos,
+                             sin, hidden.dtype, rep).transpose(1, 2)
+        v = v.reshape(b, s, self.kv_heads, self.head_dim).transpose(1, 2)
         if rep > 1:
-            k = k.repeat_interleave(rep, dim=1)
             v = v.repeat_interleave(rep, dim=1)
         out = causal_attention(q, k, v, 1.0 / math.sqrt(self.head_dim))
         return self.output(out.transpose(1, 2).reshape(b, s, self.heads * self.head_dim))
@@ -419,8 +381,9 @@ class Qwen3Layer(torch.nn.Module):
         self.mlp = Qwen3MLP(config, key + 4, device)
 
     def forward(self, hidden, cos, sin):
-        hidden = hidden + self.attention(self.input_norm(hidden), cos, sin)
-        return hidden + self.mlp(self.post_attention_norm(hidden))
+        hidden, normed = add_norm(self.post_attention_norm, hidden,
+                                  self.attention(self.input_norm(hidden), cos, sin))
+        return hidden + self.mlp(normed)
 
 
 class Qwen3TextEncoder(torch.nn.Module):

@@ -1,0 +1,155 @@
+"""The fused normalisations against float64 torch (GPU), at the edges of the
+lane layouts (rows of up to 128, 768, 2048 and 4096 elements) and of a
+workgroup's rows, and the calls that stay on the torch expressions."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from representax_amd import norms
+from representax_amd.norms import LayerNorm, RMSNorm, add_norm, head_norm_rotary
+
+DEV = "cuda:0"
+BF16, F64 = torch.bfloat16, torch.float64
+# one rounding to bf16 moves a value by at most 2^-9 of itself; f32 sums of at
+# most 4096 terms and the f32 reciprocal root are far below a quarter of that
+ONE_ROUNDING = 1.25 * 2.0 ** -9
+
+
+def _rel(a, b):
+    return float((a.to(F64) - b).norm() / b.norm().clamp_min(1e-300))
+
+
+def _module(kind, size, device=DEV, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    norm = LayerNorm(size, 1e-12, device) if kind == "layer" else RMSNorm(size, 1e-6, device)
+    with torch.no_grad():
+        for p in norm.parameters():
+            p.copy_(1.0 + 0.5 * torch.randn(size, generator=g))
+    return norm.requires_grad_(False)
+
+
+def _want(norm, t):
+    """The norm in float64; the LayerNorm takes its weights in bf16."""
+
+    if isinstance(norm, LayerNorm):
+        w, b = (p.to(BF16).to(F64) for p in (norm.weight, norm.bias))
+        return F.layer_norm(t, t.shape[-1:], w, b, norm.eps)
+    return t * torch.rsqrt(t.square().mean(-1, keepdim=True) + norm.eps) * norm.weight.to(F64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["layer", "rms"])
+@pytest.mark.parametrize("rows,size", [(1, 8), (33, 128), (17, 136), (9, 768), (7, 776),
+                                       (5, 2048), (3, 2056), (2, 4096)])
+def test_norm_and_residual_norm(kind, rows, size):
+    g = torch.Generator().manual_seed(rows * size)
+    x, r, dy, dt = (torch.randn(rows, size, generator=g).to(DEV, BF16) for _ in range(4))
+    norm = _module(kind, size)
+    x.requires_grad_(True)
+    r.requires_grad_(True)
+    y = norm(x)
+    assert "NormFn" in type(y.grad_fn).__name__
+    x64 = x.detach().to(F64).requires_grad_(True)
+    want = _want(norm, x64)
+    assert _rel(y, want) <= ONE_ROUNDING
+    (dx,) = torch.autograd.grad(y, x, dy)
+    (dx64,) = torch.autograd.grad(want, x64, dy.to(F64))
+    # a row of 8 under the LayerNorm keeps little of its gradient (two of its
+    # eight directions are projected out), still one rounding of what is left
+    assert _rel(dx, dx64) <= ONE_ROUNDING
+
+    t, y = add_norm(norm, x, r)
+    assert torch.equal(t, x + r)
+    t64 = t.detach().to(F64).requires_grad_(True)
+    want = _want(norm, t64)
+    assert _rel(y, want) <= ONE_ROUNDING
+    dx, dr = torch.autograd.grad([t, y], [x, r], [dt, dy], retain_graph=True)
+    (d64,) = torch.autograd.grad(want, t64, dy.to(F64), retain_graph=True)
+    assert torch.equal(dx, dr)
+    assert _rel(dx, d64 + dt.to(F64)) <= ONE_ROUNDING
+    # either output alone, the gradient of the norm as a transposed view
+    (only,) = torch.autograd.grad(t, x, dt, retain_graph=True)
+    assert torch.equal(only, dt)
+    (only,) = torch.autograd.grad(y, x, dy.t().contiguous().t())
+    assert _rel(only, d64) <= ONE_ROUNDING
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,s,h,d,repeat", [(1, 1, 1, 64, 1), (2, 5, 3, 128, 2), (1, 17, 8, 64, 3),
+                                            (3, 7, 16, 128, 1)])
+@pytest.mark.parametrize("weight_dtype", [torch.float32, BF16])
+def test_head_norm_with_rotation(b, s, h, d, repeat, weight_dtype):
+    g = torch.Generator().manual_seed(b * s * h)
+    x = torch.randn(b, s, h, d, generator=g).to(DEV, BF16).requires_grad_(True)
+    angle = torch.randn(1, s, d // 2, generator=g).repeat(1, 1, 2).to(DEV)
+    cos, sin = angle.cos(), angle.sin()
+    norm = _module("rms", d).to(weight_dtype)
+    y = head_norm_rotary(norm, x, cos, sin, BF16, repeat)
+    assert "HeadNormFn" in type(y.grad_fn).__name__
+    x64 = x.detach().to(F64).requires_grad_(True)
+    n = _want(norm, x64)
+    half = torch.cat((-n[..., d // 2:], n[..., :d // 2]), dim=-1)
+    want = (n * cos.to(F64)[:, :, None] + half * sin.to(F64)[:, :, None])
+    want = want.repeat_interleave(repeat, dim=2)
+    # the normalised value rounds, the rotation keeps its length, the sum rounds
+    assert _rel(y, want) <= 2 * ONE_ROUNDING
+    dy = torch.randn(b, h * repeat, s, d, generator=g).to(DEV, BF16).transpose(1, 2)
+    (dx,) = torch.autograd.grad(y, x, dy, retain_graph=True)
+    (dx64,) = torch.autograd.grad(want, x64, dy.to(F64))
+    assert _rel(dx, dx64) <= ONE_ROUNDING
+    (again,) = torch.autograd.grad(y, x, dy.contiguous())
+    assert torch.equal(dx, again)
+
+
+@pytest.mark.gpu
+def test_second_derivatives_and_torch_routes():
+    x = torch.randn(4, 64, device=DEV).to(BF16).requires_grad_(True)
+    r = torch.randn(4, 64, device=DEV).to(BF16)
+    norm = _module("rms", 64)
+    _, y = add_norm(norm, x, r)
+    (dx,) = torch.autograd.grad(y.float().square().sum(), x, create_graph=True)
+    (ddx,) = torch.autograd.grad(dx.float().square().sum(), x)
+    want = x.detach().to(F64).requires_grad_(True)
+    t = (x + r).detach().to(F64) - x.detach().to(F64)
+    (d1,) = torch.autograd.grad(_want(norm, want + t).square().sum(), want, create_graph=True)
+    (d2,) = torch.autograd.grad(d1.square().sum(), want)
+    # intermediate bf16 gradients (a handful of roundings, partly cancelling)
+    assert _rel(ddx, d2) <= 16 * ONE_ROUNDING
+
+    # weights that want a gradient, hooks, autocast, transforms, layouts
+    assert norms._row_kernel(x, norm.weight)
+    assert not norms._row_kernel(x.t(), norm.weight) and not norms._row_kernel(x[:, :60], norm.weight)
+    norm.weight.requires_grad_(True)
+    add_norm(norm, x, r)[1].sum().backward()
+    assert norm.weight.grad is not None
+    with torch.no_grad():
+        assert norms._row_kernel(x, norm.weight)
+    norm.weight.requires_grad_(False)
+    seen = []
+    handle = norm.register_forward_hook(lambda m, a, out: seen.append(a[0]))
+    t, _ = add_norm(norm, x, r)
+    assert seen and torch.equal(seen[0], t)
+    handle.remove()
+    with torch.autocast("cuda", dtype=BF16):
+        assert not norms._row_kernel(x, norm.weight)
+    rows = torch.func.vmap(norm)(x.detach())
+    assert _rel(rows, _want(norm, x.detach().to(F64))) <= 2 * ONE_ROUNDING
+    _, tangent = torch.func.jvp(lambda v: norm(v), (x.detach(),), (r,))
+    assert torch.isfinite(tangent).all()
+
+
+def test_expressions_on_the_cpu():
+    x, r = torch.randn(3, 16), torch.randn(3, 16)
+    for kind in ("layer", "rms"):
+        norm = _module(kind, 16, "cpu")
+        t, y = add_norm(norm, x, r)
+        assert torch.equal(t, x + r) and torch.equal(y, norm(x + r))
+    heads = torch.randn(2, 5, 3, 64)
+    angle = torch.randn(1, 5, 32).repeat(1, 1, 2)
+    norm = _module("rms", 64, "cpu")
+    y = head_norm_rotary(norm, heads, angle.cos(), angle.sin(), torch.float32, 2)
+    want = norms.rotate(norm(heads), angle.cos(), angle.sin()).repeat_interleave(2, dim=2)
+    assert torch.equal(y, want)
