@@ -558,6 +558,14 @@ int rpx_head_norm_backward(const void* g, int64_t stride_b, int64_t stride_s, in
                            int64_t sequence, int64_t heads, int64_t repeat, int64_t head_dim,
                            float eps, void* dx, void* stream);
 
+/* ---------------------------------------------------------------------------
+ * Compute views: up to 16 dense float32 tensors rounded to bf16 in one launch
+ * (src/representax/precision.py:111-117). Host arrays of device pointers
+ * (16-byte aligned) and element counts, read before the call returns.
+ * ------------------------------------------------------------------------- */
+int rpx_cast_many(const void* const* src, void* const* dst, const int64_t* counts, int64_t tensors,
+                  void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -30,6 +30,7 @@ from .precision import (
     active_policy,
     activation_inputs,
     compute_parameter,
+    compute_operands,
     linear_matmul,
 )
 
@@ -176,12 +177,11 @@ class QuantizedLoRALinear(torch.nn.Module):
         policy = active_policy()
         if policy is not None and policy.matrix_dtype == torch.float8_e4m3fn:
             return self._forward_fp8(value, compute_dtype)
-        a = compute_parameter(self.lora_a)
-        b = compute_parameter(self.lora_b)
+        a, b = compute_operands(self.lora_a, self.lora_b)
         x = value.to(compute_dtype)
         lead = x.shape[:-1]
         x2d = x.reshape(-1, self.input_size)
-        if x2d.dtype == torch.bfloat16 and a.dtype == torch.float32:
+        if policy is None and x2d.dtype == torch.bfloat16 and a.dtype == torch.float32:
             # no policy: jnp.matmul promotes the bf16 activations against the
             # float32 masters, so the adapter term and the output are float32
             y = ops.Int4LoRAPromotedFn.apply(x2d, a, b, self.packed_weight, self.scale_bits,
@@ -191,6 +191,8 @@ class QuantizedLoRALinear(torch.nn.Module):
                                            self.bias_bits, self.scaling, self.group_size)
         else:
             # no backward will run: the fused call alone, h kept in its scratch
+            if a.dtype != x2d.dtype:
+                a, b = ops.cast_many((a, b), x2d.dtype)
             y, _ = ops.int4lora_forward(x2d, self.packed_weight, self.scale_bits, a, b,
                                         scaling=self.scaling, group_size=self.group_size,
                                         bias_bits=self.bias_bits, need_h=False)

@@ -1820,4 +1820,31 @@ int rpx_head_norm_backward(const void* g, int64_t stride_b, int64_t stride_s, in
   return kOk;
 }
 
+// ---------------------------------------------------------------------------
+// bf16 views of float32 masters
+// ---------------------------------------------------------------------------
+int rpx_cast_many(const void* const* src, void* const* dst, const int64_t* counts, int64_t tensors,
+                  void* stream) {
+  if (tensors < 0 || tensors > kCastMany)
+    return fail_invalid("rpx_cast_many: need 0 <= tensors <= 16");
+  if (tensors == 0) return kOk;
+  if (src == nullptr || dst == nullptr || counts == nullptr)
+    return fail_invalid("rpx_cast_many: null pointer");
+  CastMany args{};
+  for (int64_t t = 0; t < tensors; ++t) {
+    if (counts[t] < 0 || counts[t] > (int64_t{1} << 36))
+      return fail_invalid("rpx_cast_many: invalid count");
+    if (counts[t] > 0 && (src[t] == nullptr || dst[t] == nullptr))
+      return fail_invalid("rpx_cast_many: null pointer");
+    if (misaligned16({src[t], dst[t]}))
+      return fail_invalid("rpx_cast_many: pointers must be 16-byte aligned");
+    args.src[t] = static_cast<const float*>(src[t]);
+    args.dst[t] = static_cast<uint16_t*>(dst[t]);
+    args.count[t] = counts[t];
+  }
+  RPX_HIP(launch_cast_many(args, static_cast<int>(tensors), static_cast<hipStream_t>(stream)),
+          "rpx_cast_many");
+  return kOk;
+}
+
 }  // extern "C"

@@ -318,4 +318,15 @@ struct HeadNormArgs {
 hipError_t launch_norm(const NormArgs& args, int kind, bool backward, hipStream_t stream);
 hipError_t launch_head_norm(const HeadNormArgs& args, bool backward, hipStream_t stream);
 
+// Conversions of up to kCastMany f32 tensors to bf16 in one launch (cast.hip);
+// 16-byte aligned pointers. `first` is filled by the launcher.
+constexpr int kCastMany = 16;
+struct CastMany {
+  const float* src[kCastMany];
+  uint16_t* dst[kCastMany];
+  int64_t count[kCastMany];
+  int64_t first[kCastMany + 1];
+};
+hipError_t launch_cast_many(CastMany args, int tensors, hipStream_t stream);
+
 }  // namespace rpx

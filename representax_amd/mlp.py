@@ -20,7 +20,8 @@ import torch.nn.functional as F
 
 from . import ops
 from .adapters import QuantizedLoRALinear
-from .precision import activation_inputs, active_compute_dtype, active_policy, compute_parameter
+from .precision import (activation_inputs, active_compute_dtype, active_policy,
+                        compute_operands, compute_parameter_dtype)
 
 
 def _fusable(value: torch.Tensor, *linears: QuantizedLoRALinear) -> bool:
@@ -33,7 +34,7 @@ def _fusable(value: torch.Tensor, *linears: QuantizedLoRALinear) -> bool:
         return False
     # bf16 adapter views; float32 masters without a policy promote the
     # adapter term to float32 (the module's own path handles that)
-    return all(compute_parameter(l.lora_a).dtype == torch.bfloat16 for l in linears)
+    return all(compute_parameter_dtype(l.lora_a) == torch.bfloat16 for l in linears)
 
 
 def _leaves(layer: QuantizedLoRALinear) -> tuple:
@@ -41,8 +42,8 @@ def _leaves(layer: QuantizedLoRALinear) -> tuple:
             layer.group_size)
 
 
-def _views(layer: QuantizedLoRALinear) -> tuple:
-    return compute_parameter(layer.lora_a), compute_parameter(layer.lora_b)
+def _adapters(*layers: QuantizedLoRALinear) -> list[torch.Tensor]:
+    return compute_operands(*(m for layer in layers for m in (layer.lora_a, layer.lora_b)))
 
 
 def gelu_mlp(value: torch.Tensor, up: torch.nn.Module, down: torch.nn.Module) -> torch.Tensor:
@@ -52,7 +53,7 @@ def gelu_mlp(value: torch.Tensor, up: torch.nn.Module, down: torch.nn.Module) ->
         return down(F.gelu(up(value)))
     x = activation_inputs(value).to(torch.bfloat16)
     lead = x.shape[:-1]
-    y = ops.Int4LoRAGeluMLPFn.apply(x.reshape(-1, up.input_size), *_views(up), *_views(down),
+    y = ops.Int4LoRAGeluMLPFn.apply(x.reshape(-1, up.input_size), *_adapters(up, down),
                                     *_leaves(up), *_leaves(down))
     return y.reshape(*lead, down.output_size)
 
@@ -65,8 +66,8 @@ def swiglu_mlp(value: torch.Tensor, gate: torch.nn.Module, up: torch.nn.Module,
         return down(F.silu(gate(value)) * up(value))
     x = activation_inputs(value).to(torch.bfloat16)
     lead = x.shape[:-1]
-    y = ops.Int4LoRASwiGLUMLPFn.apply(x.reshape(-1, up.input_size), *_views(gate), *_views(up),
-                                      *_views(down), *_leaves(gate), *_leaves(up), *_leaves(down))
+    y = ops.Int4LoRASwiGLUMLPFn.apply(x.reshape(-1, up.input_size), *_adapters(gate, up, down),
+                                      *_leaves(gate), *_leaves(up), *_leaves(down))
     return y.reshape(*lead, down.output_size)
 
 
@@ -81,14 +82,14 @@ def shared_input_projections(value: torch.Tensor, linears) -> list[torch.Tensor]
         return [layer(value) for layer in linears]
     x = activation_inputs(value).to(torch.bfloat16)
     lead = x.shape[:-1]
-    views, leaves = [], []
+    views, leaves = _adapters(*linears), []
     for layer in linears:
-        views += list(_views(layer))
         leaves += list(_leaves(layer))
     if not torch.is_grad_enabled() or not (x.requires_grad or any(v.requires_grad for v in views)):
         # inference: every projection in one call (one pair of launches for
         # all of them at small M, where a call is launch-latency bound)
         x2d = x.reshape(-1, linears[0].input_size)
+        views = ops.cast_many(views, torch.bfloat16)
         outs = ops.int4lora_forward_multi(
             x2d, [(l.packed_weight, l.scale_bits, views[2 * i], views[2 * i + 1], l.scaling,
                    l.group_size, l.bias_bits) for i, l in enumerate(linears)], need_h=False)

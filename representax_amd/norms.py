@@ -16,7 +16,8 @@ import torch
 import torch.nn.functional as F
 
 from . import _native as nat
-from .ops import BF16, F32, _aligned, _dtype_code, _on_device, _ptr, _stream
+from .ops import (BF16, F32, _aligned, _dtype_code, _on_device, _ptr, _stream, eager_calls,
+                  plain_tensor)
 
 _MAX_SIZE = 4096  # elements of a row that the kernels keep in registers
 
@@ -52,23 +53,6 @@ def rotate(value: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
 # ---------------------------------------------------------------------------
 # where the kernels apply
 # ---------------------------------------------------------------------------
-def _plain(t: torch.Tensor) -> bool:
-    """An ordinary device tensor: no subclass, no function-transform wrapper."""
-
-    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
-            and not torch._C._functorch.is_functorch_wrapped_tensor(t))
-
-
-def _eager() -> bool:
-    """Nothing watches or rewrites torch operations: the kernels may stand
-    for several of them."""
-
-    return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
-                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-                or torch.autograd.forward_ad._current_level >= 0
-                or torch.is_autocast_enabled("cuda"))
-
-
 def _dense(t: torch.Tensor) -> bool:
     return t.is_contiguous() and t.data_ptr() % 16 == 0
 
@@ -78,16 +62,17 @@ def _frozen(size: int, device, *weights: torch.Tensor) -> bool:
     dtype, none of which wants a gradient."""
 
     grad = torch.is_grad_enabled()
-    return all(_plain(w) and w.device == device and w.shape == (size,) and w.dtype in (F32, BF16)
-               and w.dtype == weights[0].dtype and _dense(w) and not (grad and w.requires_grad)
+    return all(plain_tensor(w) and w.device == device and w.shape == (size,)
+               and w.dtype in (F32, BF16) and w.dtype == weights[0].dtype and _dense(w) and not (grad and w.requires_grad)
                for w in weights)
 
 
 def _row_kernel(value: torch.Tensor, *weights: torch.Tensor) -> bool:
     size = value.shape[-1] if value.dim() else 0
-    return (_plain(value) and value.dtype == BF16 and 8 <= size <= _MAX_SIZE and size % 8 == 0
-            and 0 < value.numel() and value.numel() // size <= 1 << 31 and _dense(value)
-            and _frozen(size, value.device, *weights) and _eager())
+    return (plain_tensor(value) and value.dtype == BF16 and 8 <= size <= _MAX_SIZE
+            and size % 8 == 0 and 0 < value.numel() and value.numel() // size <= 1 << 31 and _dense(value)
+            and _frozen(size, value.device, *weights) and eager_calls()
+            and not torch.is_autocast_enabled("cuda"))
 
 
 def _unhooked(module: torch.nn.Module, cls: type) -> bool:
@@ -245,7 +230,7 @@ def add_norm(norm: torch.nn.Module, value: torch.Tensor, update: torch.Tensor):
     if kind is not None and _unhooked(norm, type(norm)):
         bias = norm.bias if kind == nat.NORM_LAYER else None
         weights = (norm.weight,) if bias is None else (norm.weight, bias)
-        if (_row_kernel(value, *weights) and _plain(update) and update.dtype == BF16
+        if (_row_kernel(value, *weights) and plain_tensor(update) and update.dtype == BF16
                 and update.shape == value.shape and update.device == value.device
                 and _dense(update)):
             return AddNormFn.apply(value, update, norm.weight, bias, kind, norm.eps)
@@ -262,7 +247,7 @@ def head_norm_rotary(norm: torch.nn.Module, heads: torch.Tensor, cos: torch.Tens
     b, s, h, d = heads.shape
     if (_unhooked(norm, RMSNorm) and d in (64, 128) and dtype == BF16
             and _row_kernel(heads, norm.weight)
-            and all(_plain(t) and t.dtype == F32 and t.device == heads.device
+            and all(plain_tensor(t) and t.dtype == F32 and t.device == heads.device
                     and t.shape == (1, s, d) and _dense(t) and not t.requires_grad
                     for t in (cos, sin))
             and h <= 65536 and repeat <= 65536):

@@ -685,16 +685,71 @@ def int4lora_backward_act(grad, x2d, packed, scale_bits, lora_a_c, lora_b_c, h, 
     return dz, dgate, d_a, d_b
 
 
+# ---------------------------------------------------------------------------
+# Compute views of float32 masters
+# ---------------------------------------------------------------------------
+CAST_MANY = 16  # tensors of one launch
+
+
+def plain_tensor(t: torch.Tensor) -> bool:
+    """An ordinary device tensor: no subclass, no function-transform wrapper."""
+
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+
+
+def eager_calls() -> bool:
+    """Nothing watches or rewrites torch operations: one kernel may stand for
+    several of them."""
+
+    return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
+def cast_many(tensors, dtype: torch.dtype) -> list[torch.Tensor]:
+    """``[t.to(dtype) for t in tensors]``; float32 to bf16 in one launch for
+    dense tensors of one device (no autograd)."""
+
+    device = tensors[0].device
+    if not (dtype == BF16 and 1 < len(tensors) <= CAST_MANY
+            and all(t.dtype == F32 and plain_tensor(t) and t.device == device
+                    and t.is_contiguous() and t.numel() and t.data_ptr() % 16 == 0
+                    for t in tensors) and eager_calls()):
+        return [t.to(dtype) for t in tensors]
+    out = [torch.empty_like(t, dtype=BF16) for t in tensors]
+    count = len(tensors)
+    pointers = ctypes.c_void_p * count
+    nat.call("rpx_cast_many", pointers(*[t.data_ptr() for t in tensors]),
+             pointers(*[t.data_ptr() for t in out]),
+             (ctypes.c_int64 * count)(*[t.numel() for t in tensors]), count,
+             _stream(_on_device(*tensors)))
+    return out
+
+
+def adapter_gradients(gradients, dtypes) -> list[torch.Tensor]:
+    """The float32 adapter gradients (bf16-rounded products under bf16
+    activations) in the dtypes of the adapters they belong to."""
+
+    if all(dtype == F32 for dtype in dtypes):
+        return list(gradients)
+    if all(dtype == BF16 for dtype in dtypes):
+        return cast_many(gradients, BF16)
+    return [d.to(dtype) for d, dtype in zip(gradients, dtypes)]
+
+
 class Int4LoRALinearFn(torch.autograd.Function):
     """Autograd node of the fused INT4 + LoRA linear on 2-D activations.
 
-    Inputs are the activations, the LoRA compute views (differentiable; their
-    gradients are the bf16-rounded products returned in the views' dtype)
-    and the frozen integer leaves.
+    Inputs are the activations, the LoRA masters or their compute views
+    (differentiable; their gradients are the products, bf16-rounded under
+    bf16 activations, in the inputs' dtype) and the frozen integer leaves.
     """
 
     @staticmethod
-    def forward(ctx, x2d, lora_a_c, lora_b_c, packed, scale_bits, bias_bits, scaling, group_size):
+    def forward(ctx, x2d, lora_a, lora_b, packed, scale_bits, bias_bits, scaling, group_size):
+        ctx.dtypes = (lora_a.dtype, lora_b.dtype)
+        lora_a_c, lora_b_c = cast_many((lora_a, lora_b), x2d.dtype)
         y, h = int4lora_forward(x2d, packed, scale_bits, lora_a_c, lora_b_c, scaling=scaling,
                                 group_size=group_size, bias_bits=bias_bits)
         ctx.save_for_backward(x2d, lora_a_c, lora_b_c, packed, scale_bits, h)
@@ -707,7 +762,7 @@ class Int4LoRALinearFn(torch.autograd.Function):
         x2d, lora_a_c, lora_b_c, packed, scale_bits, h = ctx.saved_tensors
         dx, d_a, d_b = int4lora_backward(grad_y, x2d, packed, scale_bits, lora_a_c, lora_b_c, h,
                                          scaling=ctx.scaling, group_size=ctx.group_size)
-        return (dx, d_a.to(lora_a_c.dtype), d_b.to(lora_b_c.dtype), None, None, None, None, None)
+        return (dx, *adapter_gradients((d_a, d_b), ctx.dtypes), None, None, None, None, None)
 
 
 def int4lora_forward_promoted(x2d, packed, scale_bits, lora_a, lora_b, *, scaling: float,
@@ -785,13 +840,16 @@ class Int4LoRAGeluMLPFn(torch.autograd.Function):
     the up projection's GEMM epilogue and its backward in the down
     projection's dx epilogue (bert/model.py:249).
 
-    Per linear: LoRA compute views (a, b), then packed, scale_bits,
+    Per linear: LoRA masters or compute views (a, b), then packed, scale_bits,
     bias_bits, scaling, group_size.
     """
 
     @staticmethod
     def forward(ctx, x2d, up_a, up_b, down_a, down_b, up_packed, up_scales, up_bias, up_scaling,
                 up_group, down_packed, down_scales, down_bias, down_scaling, down_group):
+        adapters = (up_a, up_b, down_a, down_b)
+        ctx.dtypes = [t.dtype for t in adapters]
+        up_a, up_b, down_a, down_b = cast_many(adapters, x2d.dtype)
         act, z, h_up = int4lora_forward_act(x2d, up_packed, up_scales, up_a, up_b,
                                             activation="gelu", scaling=up_scaling,
                                             group_size=up_group, bias_bits=up_bias)
@@ -813,8 +871,8 @@ class Int4LoRAGeluMLPFn(torch.autograd.Function):
             z=z, scaling=down_scaling, group_size=down_group)
         dx, d_up_a, d_up_b = int4lora_backward(dz, x2d, up_packed, up_scales, up_a, up_b, h_up,
                                                scaling=up_scaling, group_size=up_group)
-        return (dx, d_up_a.to(up_a.dtype), d_up_b.to(up_b.dtype), d_down_a.to(down_a.dtype),
-                d_down_b.to(down_b.dtype)) + (None,) * 10
+        return (dx, *adapter_gradients((d_up_a, d_up_b, d_down_a, d_down_b), ctx.dtypes)) \
+            + (None,) * 10
 
 
 class Int4LoRASwiGLUMLPFn(torch.autograd.Function):
@@ -827,6 +885,9 @@ class Int4LoRASwiGLUMLPFn(torch.autograd.Function):
     def forward(ctx, x2d, gate_a, gate_b, up_a, up_b, down_a, down_b, gate_packed, gate_scales,
                 gate_bias, gate_scaling, gate_group, up_packed, up_scales, up_bias, up_scaling,
                 up_group, down_packed, down_scales, down_bias, down_scaling, down_group):
+        adapters = (gate_a, gate_b, up_a, up_b, down_a, down_b)
+        ctx.dtypes = [t.dtype for t in adapters]
+        gate_a, gate_b, up_a, up_b, down_a, down_b = cast_many(adapters, x2d.dtype)
         g, h_gate = int4lora_forward(x2d, gate_packed, gate_scales, gate_a, gate_b,
                                      scaling=gate_scaling, group_size=gate_group,
                                      bias_bits=gate_bias)
@@ -857,9 +918,8 @@ class Int4LoRASwiGLUMLPFn(torch.autograd.Function):
         dx, _, d_gate_a, d_gate_b = int4lora_backward_act(
             dg, x2d, gate_packed, gate_scales, gate_a, gate_b, h_gate, activation="add", z=dx_up,
             scaling=gate_scaling, group_size=gate_group)
-        return (dx, d_gate_a.to(gate_a.dtype), d_gate_b.to(gate_b.dtype),
-                d_up_a.to(up_a.dtype), d_up_b.to(up_b.dtype), d_down_a.to(down_a.dtype),
-                d_down_b.to(down_b.dtype)) + (None,) * 15
+        gradients = (d_gate_a, d_gate_b, d_up_a, d_up_b, d_down_a, d_down_b)
+        return (dx, *adapter_gradients(gradients, ctx.dtypes)) + (None,) * 15
 
 
 class Int4LoRASharedInputFn(torch.autograd.Function):
@@ -870,13 +930,14 @@ class Int4LoRASharedInputFn(torch.autograd.Function):
     gradient after the first is added to the running sum in its dx GEMM's
     epilogue (bf16, in projection order) instead of by a separate pass.
 
-    Arguments: x2d, the count n, the n pairs of LoRA compute views, then per
+    Arguments: x2d, the count n, the n pairs of LoRA masters or views, then per
     linear packed, scale_bits, bias_bits, scaling, group_size.
     """
 
     @staticmethod
     def forward(ctx, x2d, n, *args):
-        views = args[:2 * n]
+        ctx.dtypes = [t.dtype for t in args[:2 * n]]
+        views = cast_many(args[:2 * n], x2d.dtype)
         leaves = args[2 * n:]
         outs, hs = [], []
         if x2d.dim() == 2 and x2d.shape[0] > SHARED_OUTPUT_ROWS:
@@ -923,8 +984,8 @@ class Int4LoRASharedInputFn(torch.autograd.Function):
                 dx, _, d_a, d_b = int4lora_backward_act(
                     g, x2d, packed[i], scales[i], a, b, hs[i], activation="add", z=dx,
                     scaling=scaling, group_size=group)
-            dviews += [d_a.to(a.dtype), d_b.to(b.dtype)]
-        return (dx, None, *dviews) + (None,) * (5 * n)
+            dviews += [d_a, d_b]
+        return (dx, None, *adapter_gradients(dviews, ctx.dtypes)) + (None,) * (5 * n)
 
 
 # ---------------------------------------------------------------------------

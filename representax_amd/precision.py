@@ -284,6 +284,26 @@ def compute_parameter(value: torch.Tensor) -> torch.Tensor:
     return value.to(policy.compute_dtype)
 
 
+def compute_operands(*values: torch.Tensor) -> list[torch.Tensor]:
+    """``[compute_parameter(v) for v in values]`` for the fused calls, which
+    cast the float32 masters themselves: those stay as they are under bf16
+    compute, so that no cast (nor its transpose) runs on its own."""
+
+    policy = _ACTIVE_PRECISION.get()
+    views = _COMPUTE_VIEWS.get()
+    if policy is None or policy.compute_dtype != torch.bfloat16 or views is not None:
+        return [compute_parameter(v) for v in values]
+    kept = (torch.float32, torch.bfloat16)
+    return [v if v.dtype in kept else v.to(torch.bfloat16) for v in values]
+
+
+def compute_parameter_dtype(value: torch.Tensor) -> torch.dtype:
+    """The dtype of ``compute_parameter(value)``."""
+
+    policy = _ACTIVE_PRECISION.get()
+    return value.dtype if policy is None else policy.compute_dtype
+
+
 def active_compute_dtype(fallback: torch.dtype) -> torch.dtype:
     """Active policy's compute dtype, else ``fallback`` (precision.py:120-124)."""
 
