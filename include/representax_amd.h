@@ -540,23 +540,29 @@ int rpx_norm_backward(const void* dy, const void* dsum, const void* t, const voi
                       int weight_dtype, int64_t rows, int64_t size, float eps, int kind, void* dx,
                       void* stream);
 
-/* y[token, h * repeat + j] = rotate(rms_norm(x[token, h])) for j < repeat:
- * x [tokens, heads, head_dim], y [tokens, heads * repeat, head_dim], cosines and
- * sines f32 [sequence, head_dim], the position of a token being its index
- * modulo `sequence`. Requires head_dim 64 or 128. */
-int rpx_head_norm_forward(const void* x, const void* weight, int weight_dtype,
-                          const void* cosines, const void* sines, int64_t tokens,
-                          int64_t sequence, int64_t heads, int64_t repeat, int64_t head_dim,
-                          float eps, void* y, void* stream);
+/* Up to three sets of heads of one layer (queries, keys, values) in a launch.
+ * Forward: out[token, h * repeat + j] = rotate(rms_norm(x[token, h])) for
+ * j < repeat, or x[token, h] itself where weight is null; x [tokens, heads,
+ * head_dim], out [tokens, heads * repeat, head_dim]; cosines and sines f32
+ * [sequence, head_dim], the position of a token being its index modulo
+ * `sequence`. Backward: out [tokens, heads, head_dim] = the gradient of x for
+ * the gradient g of that output, whose element (b, s, h, d) lies at b * stride_b
+ * + s * stride_s + h * stride_h + d (strides multiples of 8). Requires head_dim
+ * 64 or 128. */
+typedef struct rpx_head_part {
+  const void* x;
+  const void* weight;
+  const void* g;
+  void* out;
+  int64_t stride_b, stride_s, stride_h;
+  int64_t heads, repeat;
+  int weight_dtype;
+  float eps;
+} rpx_head_part;
 
-/* dx [tokens, heads, head_dim] for the gradient g of y, whose element
- * (b, s, h, d) lies at b * stride_b + s * stride_s + h * stride_h + d
- * (multiples of 8). */
-int rpx_head_norm_backward(const void* g, int64_t stride_b, int64_t stride_s, int64_t stride_h,
-                           const void* x, const void* weight, int weight_dtype,
-                           const void* cosines, const void* sines, int64_t tokens,
-                           int64_t sequence, int64_t heads, int64_t repeat, int64_t head_dim,
-                           float eps, void* dx, void* stream);
+int rpx_head_norm(const rpx_head_part* parts, int64_t count, const void* cosines,
+                  const void* sines, int64_t tokens, int64_t sequence, int64_t head_dim,
+                  int backward, void* stream);
 
 /* ---------------------------------------------------------------------------
  * Compute views: up to 16 dense float32 tensors rounded to bf16 in one launch

@@ -144,14 +144,17 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "rpx_cast_many": (_int, [_p, _p, _p, _i64, _p]),
     "rpx_norm_forward": (_int, [_p, _p, _p, _p, _int, _i64, _i64, _f32, _int, _p, _p, _p]),
     "rpx_norm_backward": (_int, [_p, _p, _p, _p, _int, _i64, _i64, _f32, _int, _p, _p]),
-    "rpx_head_norm_forward": (
-        _int, [_p, _p, _int, _p, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p, _p]
-    ),
-    "rpx_head_norm_backward": (
-        _int,
-        [_p, _i64, _i64, _i64, _p, _p, _int, _p, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p, _p],
-    ),
+    "rpx_head_norm": (_int, [_p, _i64, _p, _p, _i64, _i64, _i64, _int, _p]),
 }
+
+
+class HeadPart(ctypes.Structure):
+    """``rpx_head_part`` of include/representax_amd.h."""
+
+    _fields_ = [(name, ctypes.c_void_p) for name in ("x", "weight", "g", "out")]
+    _fields_ += [(name, ctypes.c_int64)
+                 for name in ("stride_b", "stride_s", "stride_h", "heads", "repeat")]
+    _fields_ += [("weight_dtype", ctypes.c_int), ("eps", ctypes.c_float)]
 
 
 class Int4LoraProjection(ctypes.Structure):

@@ -1743,80 +1743,51 @@ int rpx_norm_backward(const void* dy, const void* dsum, const void* t, const voi
   return kOk;
 }
 
-static int check_head_norm(int weight_dtype, int64_t tokens, int64_t sequence, int64_t heads,
-                           int64_t repeat, int64_t head_dim, const char* who) {
-  RPX_TRY(check_dtype(weight_dtype));
-  if (tokens < 0 || sequence < 1 || heads < 1 || heads > 65536 || repeat < 1 || repeat > 65536 ||
-      tokens > (int64_t{1} << 31) / heads)
-    return fail_invalid(std::string(who) + ": invalid extents");
+int rpx_head_norm(const rpx_head_part* parts, int64_t count, const void* cosines,
+                  const void* sines, int64_t tokens, int64_t sequence, int64_t head_dim,
+                  int backward, void* stream) {
+  const std::string who = "rpx_head_norm";
+  if (count < 0 || count > kHeadParts) return fail_invalid(who + ": need 0 <= parts <= 3");
+  if (tokens < 0 || sequence < 1) return fail_invalid(who + ": invalid extents");
   if (head_dim != 64 && head_dim != 128)
-    return fail_invalid(std::string(who) + ": head_dim must be 64 or 128");
-  return kOk;
-}
-
-int rpx_head_norm_forward(const void* x, const void* weight, int weight_dtype,
-                          const void* cosines, const void* sines, int64_t tokens,
-                          int64_t sequence, int64_t heads, int64_t repeat, int64_t head_dim,
-                          float eps, void* y, void* stream) {
-  RPX_TRY(check_head_norm(weight_dtype, tokens, sequence, heads, repeat, head_dim,
-                          "rpx_head_norm_forward"));
-  if (tokens == 0) return kOk;
-  if (x == nullptr || weight == nullptr || cosines == nullptr || sines == nullptr || y == nullptr)
-    return fail_invalid("rpx_head_norm_forward: null pointer");
-  if (misaligned16({x, weight, cosines, sines, y}))
-    return fail_invalid("rpx_head_norm_forward: pointers must be 16-byte aligned");
+    return fail_invalid(who + ": head_dim must be 64 or 128");
+  if (count == 0 || tokens == 0) return kOk;
+  if (parts == nullptr || cosines == nullptr || sines == nullptr)
+    return fail_invalid(who + ": null pointer");
+  if (misaligned16({cosines, sines}))
+    return fail_invalid(who + ": pointers must be 16-byte aligned");
   HeadNormArgs args{};
-  args.x = static_cast<const uint16_t*>(x);
-  args.weight = weight;
-  args.weight_dtype = weight_dtype;
   args.cosines = static_cast<const float*>(cosines);
   args.sines = static_cast<const float*>(sines);
   args.tokens = tokens;
   args.sequence = sequence;
-  args.heads = static_cast<int>(heads);
-  args.repeat = static_cast<int>(repeat);
   args.head_dim = static_cast<int>(head_dim);
-  args.eps = eps;
-  args.out = static_cast<uint16_t*>(y);
-  RPX_HIP(launch_head_norm(args, false, static_cast<hipStream_t>(stream)),
-          "rpx_head_norm_forward");
-  return kOk;
-}
-
-int rpx_head_norm_backward(const void* g, int64_t stride_b, int64_t stride_s, int64_t stride_h,
-                           const void* x, const void* weight, int weight_dtype,
-                           const void* cosines, const void* sines, int64_t tokens,
-                           int64_t sequence, int64_t heads, int64_t repeat, int64_t head_dim,
-                           float eps, void* dx, void* stream) {
-  RPX_TRY(check_head_norm(weight_dtype, tokens, sequence, heads, repeat, head_dim,
-                          "rpx_head_norm_backward"));
-  if (tokens == 0) return kOk;
-  if (g == nullptr || x == nullptr || weight == nullptr || cosines == nullptr ||
-      sines == nullptr || dx == nullptr)
-    return fail_invalid("rpx_head_norm_backward: null pointer");
-  if (misaligned16({g, x, weight, cosines, sines, dx}) || stride_b % 8 != 0 || stride_s % 8 != 0 ||
-      stride_h % 8 != 0)
-    return fail_invalid("rpx_head_norm_backward: pointers must be 16-byte aligned, strides "
-                        "multiples of 8");
-  HeadNormArgs args{};
-  args.g = static_cast<const uint16_t*>(g);
-  args.stride_b = stride_b;
-  args.stride_s = stride_s;
-  args.stride_h = stride_h;
-  args.x = static_cast<const uint16_t*>(x);
-  args.weight = weight;
-  args.weight_dtype = weight_dtype;
-  args.cosines = static_cast<const float*>(cosines);
-  args.sines = static_cast<const float*>(sines);
-  args.tokens = tokens;
-  args.sequence = sequence;
-  args.heads = static_cast<int>(heads);
-  args.repeat = static_cast<int>(repeat);
-  args.head_dim = static_cast<int>(head_dim);
-  args.eps = eps;
-  args.out = static_cast<uint16_t*>(dx);
-  RPX_HIP(launch_head_norm(args, true, static_cast<hipStream_t>(stream)),
-          "rpx_head_norm_backward");
+  for (int64_t p = 0; p < count; ++p) {
+    const rpx_head_part& in = parts[p];
+    if (in.weight != nullptr) RPX_TRY(check_dtype(in.weight_dtype));
+    if (in.heads < 1 || in.heads > 65536 || in.repeat < 1 || in.repeat > 65536 ||
+        tokens > (int64_t{1} << 31) / in.heads)
+      return fail_invalid(who + ": invalid extents");
+    if (in.x == nullptr || in.out == nullptr || (backward != 0 && in.g == nullptr))
+      return fail_invalid(who + ": null pointer");
+    if (misaligned16({in.x, in.weight, in.g, in.out}) || in.stride_b % 8 != 0 ||
+        in.stride_s % 8 != 0 || in.stride_h % 8 != 0)
+      return fail_invalid(who + ": pointers must be 16-byte aligned, strides multiples of 8");
+    args.part[p] = HeadPart{static_cast<const uint16_t*>(in.x),
+                            in.weight,
+                            static_cast<const uint16_t*>(in.g),
+                            in.stride_b,
+                            in.stride_s,
+                            in.stride_h,
+                            static_cast<uint16_t*>(in.out),
+                            in.eps,
+                            in.weight_dtype,
+                            static_cast<int>(in.heads),
+                            static_cast<int>(in.repeat)};
+  }
+  RPX_HIP(launch_head_norm(args, static_cast<int>(count), backward != 0,
+                           static_cast<hipStream_t>(stream)),
+          "rpx_head_norm");
   return kOk;
 }
 

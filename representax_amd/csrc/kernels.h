@@ -301,22 +301,27 @@ struct NormArgs {
   uint16_t* y;    // backward: the gradient of the row
 };
 
-struct HeadNormArgs {
-  const uint16_t* g;  // backward: the gradient of the rotated heads and its strides
-  int64_t stride_b, stride_s, stride_h;
+constexpr int kHeadParts = 3;
+struct HeadPart {
   const uint16_t* x;  // [tokens, heads, head_dim]
-  const void* weight;
-  int weight_dtype;
+  const void* weight;  // nullptr: the heads are only repeated
+  const uint16_t* g;   // backward: the gradient of the output, by its strides
+  int64_t stride_b, stride_s, stride_h;
+  uint16_t* out;
+  float eps;
+  int weight_dtype, heads, repeat;
+};
+struct HeadNormArgs {
+  HeadPart part[kHeadParts];
   const float* cosines;  // [sequence, head_dim]
   const float* sines;
   int64_t tokens, sequence;
-  int heads, repeat, head_dim;  // head_dim 64 or 128
-  float eps;
-  uint16_t* out;
+  int head_dim;  // 64 or 128
+  int64_t first[kHeadParts + 1];  // filled by the launcher
 };
 
 hipError_t launch_norm(const NormArgs& args, int kind, bool backward, hipStream_t stream);
-hipError_t launch_head_norm(const HeadNormArgs& args, bool backward, hipStream_t stream);
+hipError_t launch_head_norm(HeadNormArgs args, int parts, bool backward, hipStream_t stream);
 
 // Conversions of up to kCastMany f32 tensors to bf16 in one launch (cast.hip);
 // 16-byte aligned pointers. `first` is filled by the launcher.

@@ -125,23 +125,28 @@ __global__ void __launch_bounds__(kThreads)
       unpack8(t, v[c]);
     }
   }
+  // the weights' loads are in flight while the statistics are summed
+  float g[C][8], h[KIND == kNormLayer ? C : 1][8];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int e = (c * L + lane) * 8;
+    if (e >= size) continue;
+    load_weight8<KIND == kNormLayer>(w, w_dtype, e, g[c]);
+    if constexpr (KIND == kNormLayer) load_weight8<true>(b, w_dtype, e, h[c]);
+  }
   float mean, rstd;
   row_stats<KIND, L, C>(v, lane, size, eps, &mean, &rstd);
 #pragma unroll
   for (int c = 0; c < C; ++c) {
     const int e = (c * L + lane) * 8;
     if (e >= size) continue;
-    float g[8];
-    load_weight8<KIND == kNormLayer>(w, w_dtype, e, g);
     if constexpr (KIND == kNormLayer) {
-      float h[8];
-      load_weight8<true>(b, w_dtype, e, h);
 #pragma unroll
       for (int i = 0; i < 8; ++i)
-        v[c][i] = __builtin_fmaf((v[c][i] - mean) * rstd, g[i], h[i]);
+        v[c][i] = __builtin_fmaf((v[c][i] - mean) * rstd, g[c][i], h[c][i]);
     } else {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[c][i] = v[c][i] * rstd * g[i];
+      for (int i = 0; i < 8; ++i) v[c][i] = v[c][i] * rstd * g[c][i];
     }
     *reinterpret_cast<u32x4_t*>(y + base + e) = pack8(v[c]);
   }
@@ -219,82 +224,91 @@ __global__ void __launch_bounds__(kThreads)
 }
 
 // Heads of D = 8 * L elements, one per L lanes: lane l holds the elements
-// 8 l .. 8 l + 7, so the rotation's other half is lane l ^ (L / 2).
-// x [tokens, heads, D] dense; y [tokens, heads * repeat, D] dense, head h
-// written `repeat` times (the keys of grouped queries).
-template <int L>
-__global__ void __launch_bounds__(kThreads)
-    k_head_norm_fwd(const uint16_t* __restrict__ x, const void* __restrict__ w, int w_dtype,
-                    const float* __restrict__ cosines, const float* __restrict__ sines,
-                    int64_t tokens, int64_t sequence, int heads, int repeat, float eps,
-                    uint16_t* __restrict__ y) {
-  constexpr int kD = 8 * L;
-  const int lane = threadIdx.x & (L - 1);
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * (kThreads / L) + threadIdx.x / L;
-  if (row >= tokens * heads) return;
-  const int64_t token = row / heads;
-  const int e = 8 * lane;
-  float v[1][8], wv[8], cs[8], sn[8];
-  load8(x + row * kD + e, v[0]);
-  load_weight8<false>(w, w_dtype, e, wv);
-  const int64_t at = (token % sequence) * kD + e;
-  load_weight8<false>(cosines + at, kF32, 0, cs);
-  load_weight8<false>(sines + at, kF32, 0, sn);
-  float mean, rstd;
-  row_stats<kNormRms, L, 1>(v, lane, kD, eps, &mean, &rstd);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float n = round_bf16(v[0][i] * rstd * wv[i]);
-    const float other = __shfl_xor(n, L / 2, 64);
-    v[0][i] = n * cs[i] + (lane < L / 2 ? -other : other) * sn[i];
-  }
-  const u32x4_t out = pack8(v[0]);
-  for (int j = 0; j < repeat; ++j)
-    *reinterpret_cast<u32x4_t*>(y + (row * repeat + j) * kD + e) = out;
+// 8 l .. 8 l + 7, so the rotation's other half is lane l ^ (L / 2). The parts
+// (queries, keys and the values that only repeat) share a launch: blocks
+// [first[p], first[p + 1]) are part p's. x [tokens, heads, D] dense; y [tokens,
+// heads * repeat, D] dense, head h written `repeat` times.
+__device__ __forceinline__ int head_part(const HeadNormArgs& a) {
+  int p = 0;
+  while (static_cast<int64_t>(blockIdx.x) >= a.first[p + 1]) ++p;
+  return p;
 }
 
-// dx; g's element (b, s, h, d) at b * sb + s * ss + h * sh + d.
 template <int L>
-__global__ void __launch_bounds__(kThreads)
-    k_head_norm_bwd(const uint16_t* __restrict__ g, int64_t sb, int64_t ss, int64_t sh,
-                    const uint16_t* __restrict__ x, const void* __restrict__ w, int w_dtype,
-                    const float* __restrict__ cosines, const float* __restrict__ sines,
-                    int64_t tokens, int64_t sequence, int heads, int repeat, float eps,
-                    uint16_t* __restrict__ dx) {
+__global__ void __launch_bounds__(kThreads) k_head_norm_fwd(HeadNormArgs a) {
   constexpr int kD = 8 * L;
+  const int p = head_part(a);
+  const HeadPart& part = a.part[p];
   const int lane = threadIdx.x & (L - 1);
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * (kThreads / L) + threadIdx.x / L;
-  if (row >= tokens * heads) return;
-  const int64_t token = row / heads;
-  const int64_t s = token % sequence;
-  const int64_t head = row % heads;
+  const int64_t row = (blockIdx.x - a.first[p]) * (kThreads / L) + threadIdx.x / L;
+  if (row >= a.tokens * part.heads) return;
+  const int64_t token = row / part.heads;
   const int e = 8 * lane;
-  float v[1][8], dv[1][8], wv[8], cs[8], sn[8];
-  load8(x + row * kD + e, v[0]);
-  load_weight8<false>(w, w_dtype, e, wv);
-  load_weight8<false>(cosines + s * kD + e, kF32, 0, cs);
-  load_weight8<false>(sines + s * kD + e, kF32, 0, sn);
+  u32x4_t out = *reinterpret_cast<const u32x4_t*>(part.x + row * kD + e);
+  if (part.weight != nullptr) {
+    float v[1][8], wv[8], cs[8], sn[8];
+    unpack8(out, v[0]);
+    load_weight8<false>(part.weight, part.weight_dtype, e, wv);
+    const int64_t at = (token % a.sequence) * kD + e;
+    load_weight8<false>(a.cosines + at, kF32, 0, cs);
+    load_weight8<false>(a.sines + at, kF32, 0, sn);
+    float mean, rstd;
+    row_stats<kNormRms, L, 1>(v, lane, kD, part.eps, &mean, &rstd);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float n = round_bf16(v[0][i] * rstd * wv[i]);
+      const float other = __shfl_xor(n, L / 2, 64);
+      v[0][i] = n * cs[i] + (lane < L / 2 ? -other : other) * sn[i];
+    }
+    out = pack8(v[0]);
+  }
+  for (int j = 0; j < part.repeat; ++j)
+    *reinterpret_cast<u32x4_t*>(part.out + (row * part.repeat + j) * kD + e) = out;
+}
+
+// dx; g's element (b, s, h, d) at b * stride_b + s * stride_s + h * stride_h + d.
+template <int L>
+__global__ void __launch_bounds__(kThreads) k_head_norm_bwd(HeadNormArgs a) {
+  constexpr int kD = 8 * L;
+  const int p = head_part(a);
+  const HeadPart& part = a.part[p];
+  const int lane = threadIdx.x & (L - 1);
+  const int64_t row = (blockIdx.x - a.first[p]) * (kThreads / L) + threadIdx.x / L;
+  if (row >= a.tokens * part.heads) return;
+  const int64_t token = row / part.heads;
+  const int64_t s = token % a.sequence;
+  const int64_t head = row % part.heads;
+  const int e = 8 * lane;
+  float dv[1][8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) dv[0][i] = 0.0f;
-  const uint16_t* gr = g + (token / sequence) * sb + s * ss + head * repeat * sh + e;
-  for (int j = 0; j < repeat; ++j) {
-    float a[8];
-    load8(gr + j * sh, a);
+  const uint16_t* gr = part.g + (token / a.sequence) * part.stride_b + s * part.stride_s +
+                       head * part.repeat * part.stride_h + e;
+  for (int j = 0; j < part.repeat; ++j) {
+    float t[8];
+    load8(gr + j * part.stride_h, t);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) dv[0][i] += a[i];
+    for (int i = 0; i < 8; ++i) dv[0][i] += t[i];
   }
-  float mean, rstd;
-  row_stats<kNormRms, L, 1>(v, lane, kD, eps, &mean, &rstd);
+  if (part.weight != nullptr) {
+    float v[1][8], wv[8], cs[8], sn[8];
+    load8(part.x + row * kD + e, v[0]);
+    load_weight8<false>(part.weight, part.weight_dtype, e, wv);
+    load_weight8<false>(a.cosines + s * kD + e, kF32, 0, cs);
+    load_weight8<false>(a.sines + s * kD + e, kF32, 0, sn);
+    float mean, rstd;
+    row_stats<kNormRms, L, 1>(v, lane, kD, part.eps, &mean, &rstd);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    // the rotation's transpose: the other half's gradient times its sine
-    const float other = __shfl_xor(dv[0][i] * sn[i], L / 2, 64);
-    const float dn = dv[0][i] * cs[i] + (lane < L / 2 ? other : -other);
-    dv[0][i] = dn * wv[i];
-    v[0][i] *= rstd;
+    for (int i = 0; i < 8; ++i) {
+      // the rotation's transpose: the other half's gradient times its sine
+      const float other = __shfl_xor(dv[0][i] * sn[i], L / 2, 64);
+      const float dn = dv[0][i] * cs[i] + (lane < L / 2 ? other : -other);
+      dv[0][i] = dn * wv[i];
+      v[0][i] *= rstd;
+    }
+    row_gradient<kNormRms, L, 1>(v, dv, kD, rstd);
   }
-  row_gradient<kNormRms, L, 1>(v, dv, kD, rstd);
-  *reinterpret_cast<u32x4_t*>(dx + row * kD + e) = pack8(dv[0]);
+  *reinterpret_cast<u32x4_t*>(part.out + row * kD + e) = pack8(dv[0]);
 }
 
 // Lanes a row and chunks a lane: the fewest that hold the row, so that short
@@ -340,26 +354,16 @@ hipError_t launch_norm(const NormArgs& a, int kind, bool backward, hipStream_t s
   return hipGetLastError();
 }
 
-hipError_t launch_head_norm(const HeadNormArgs& a, bool backward, hipStream_t stream) {
-  if (a.tokens <= 0) return hipSuccess;
+hipError_t launch_head_norm(HeadNormArgs a, int parts, bool backward, hipStream_t stream) {
   const int lanes = a.head_dim / 8;
-  const dim3 grid(static_cast<unsigned>(ceil_div(a.tokens * a.heads, kThreads / lanes)));
-#define RPX_HEAD(L)                                                                             \
-  do {                                                                                          \
-    if (backward)                                                                               \
-      hipLaunchKernelGGL(k_head_norm_bwd<L>, grid, dim3(kThreads), 0, stream, a.g, a.stride_b,  \
-                         a.stride_s, a.stride_h, a.x, a.weight, a.weight_dtype, a.cosines,      \
-                         a.sines, a.tokens, a.sequence, a.heads, a.repeat, a.eps, a.out);       \
-    else                                                                                        \
-      hipLaunchKernelGGL(k_head_norm_fwd<L>, grid, dim3(kThreads), 0, stream, a.x, a.weight,    \
-                         a.weight_dtype, a.cosines, a.sines, a.tokens, a.sequence, a.heads,     \
-                         a.repeat, a.eps, a.out);                                               \
-  } while (0)
-  if (a.head_dim == 128)
-    RPX_HEAD(16);
-  else
-    RPX_HEAD(8);
-#undef RPX_HEAD
+  a.first[0] = 0;
+  for (int p = 0; p < parts; ++p)
+    a.first[p + 1] = a.first[p] + ceil_div(a.tokens * a.part[p].heads, kThreads / lanes);
+  if (a.first[parts] == 0) return hipSuccess;
+  const auto kernel = a.head_dim == 128 ? (backward ? k_head_norm_bwd<16> : k_head_norm_fwd<16>)
+                                        : (backward ? k_head_norm_bwd<8> : k_head_norm_fwd<8>);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(a.first[parts])), dim3(kThreads), 0,
+                     stream, a);
   return hipGetLastError();
 }
 

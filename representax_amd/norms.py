@@ -43,11 +43,13 @@ def _rotate_half(value: torch.Tensor) -> torch.Tensor:
     return torch.cat((-second, first), dim=-1)
 
 
-def rotate(value: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
+def rotate(value: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+           dtype: torch.dtype | None = None) -> torch.Tensor:
     """The rotary rotation of ``[B, S, H, D]`` by ``[1, S, D]`` angles, in float32."""
 
     cos, sin = cos[:, :, None], sin[:, :, None]
-    return (value.float() * cos + _rotate_half(value.float()) * sin).to(value.dtype)
+    value, dtype = value.float(), dtype or value.dtype
+    return (value * cos + _rotate_half(value) * sin).to(dtype)
 
 
 # ---------------------------------------------------------------------------
@@ -159,37 +161,59 @@ class AddNormFn(torch.autograd.Function):
 
 
 class HeadNormFn(torch.autograd.Function):
-    """Per-head RMSNorm with a frozen weight, the rotary rotation, and each
-    head repeated ``repeat`` times: ``[B, S, H, D] -> [B, S, H * repeat, D]``."""
+    """A layer's queries, keys and values in one launch: per-head RMSNorm with
+    a frozen weight and the rotary rotation (where there is a weight), each
+    head repeated: ``[B, S, H, D] -> [B, S, H * repeat, D]``.
+
+    Arguments: cos, sin, a tuple of (eps, repeat) per part, then per part x
+    and its weight or None.
+    """
 
     @staticmethod
-    def forward(ctx, x, weight, cos, sin, eps, repeat):
-        device = _on_device(x, weight, cos, sin)
-        b, s, h, d = x.shape
-        y = torch.empty((b, s, h * repeat, d), dtype=BF16, device=device)
-        nat.call("rpx_head_norm_forward", _ptr(x), _ptr(weight), _dtype_code(weight.dtype),
-                 _ptr(cos), _ptr(sin), b * s, s, h, repeat, d, float(eps), _ptr(y),
-                 _stream(device))
-        ctx.save_for_backward(x, weight, cos, sin)
-        ctx.eps, ctx.repeat = eps, repeat
-        return y
+    def forward(ctx, cos, sin, cfg, *operands):
+        xs, weights = operands[::2], operands[1::2]
+        b, s, _, d = xs[0].shape
+        ctx.cfg = cfg
+        ctx.save_for_backward(cos, sin, *operands)
+        outs = [torch.empty((b, s, x.shape[2] * repeat, d), dtype=BF16, device=x.device)
+                for x, (_, repeat) in zip(xs, cfg)]
+        _head_norm(cos, sin, cfg, xs, weights, None, outs)
+        return tuple(outs)
 
     @staticmethod
-    def backward(ctx, g):
-        x, weight, cos, sin = ctx.saved_tensors
+    def backward(ctx, *grads):
+        cos, sin, *operands = ctx.saved_tensors
+        xs, weights = operands[::2], operands[1::2]
         if torch.is_grad_enabled():  # create_graph: the gradient is differentiated again
-            y = rotate(rms_norm(x, weight, ctx.eps), cos, sin)
-            y = y.repeat_interleave(ctx.repeat, dim=2)
-            return torch.autograd.grad(y, x, g, create_graph=True)[0], None, None, None, None, None
-        device = _on_device(x, g)
-        b, s, h, d = x.shape
-        if g.stride(3) != 1 or any(n % 8 for n in g.stride()[:3]) or g.data_ptr() % 16:
-            g = _aligned(g)
-        dx = torch.empty_like(x)
-        nat.call("rpx_head_norm_backward", _ptr(g), g.stride(0), g.stride(1), g.stride(2), _ptr(x),
-                 _ptr(weight), _dtype_code(weight.dtype), _ptr(cos), _ptr(sin), b * s, s, h,
-                 ctx.repeat, d, float(ctx.eps), _ptr(dx), _stream(device))
-        return dx, None, None, None, None, None
+            found = []
+            for x, w, g, (eps, repeat) in zip(xs, weights, grads, ctx.cfg):
+                y = x if w is None else rotate(rms_norm(x, w, eps), cos, sin)
+                y = y.repeat_interleave(repeat, dim=2)
+                found += [torch.autograd.grad(y, x, g, create_graph=True)[0]
+                          if x.requires_grad else None, None]
+            return (None, None, None, *found)
+        grads = [g if g.stride(3) == 1 and not any(n % 8 for n in g.stride()[:3])
+                 and g.data_ptr() % 16 == 0 else _aligned(g) for g in grads]
+        outs = [torch.empty_like(x) for x in xs]
+        _head_norm(cos, sin, ctx.cfg, xs, weights, grads, outs)
+        return (None, None, None, *(t for dx in outs for t in (dx, None)))
+
+
+def _head_norm(cos, sin, cfg, xs, weights, grads, outs) -> None:
+    device = _on_device(cos, sin, *xs, *weights)
+    b, s, _, d = xs[0].shape
+    parts = (nat.HeadPart * len(xs))()
+    for i, (x, w, (eps, repeat)) in enumerate(zip(xs, weights, cfg)):
+        part = parts[i]
+        part.x, part.out = x.data_ptr(), outs[i].data_ptr()
+        part.heads, part.repeat, part.eps = x.shape[2], repeat, eps
+        if w is not None:
+            part.weight, part.weight_dtype = w.data_ptr(), _dtype_code(w.dtype)
+        if grads is not None:
+            part.g = grads[i].data_ptr()
+            part.stride_b, part.stride_s, part.stride_h, _ = grads[i].stride()
+    nat.call("rpx_head_norm", parts, len(xs), _ptr(cos), _ptr(sin), b * s, s, d,
+             int(grads is not None), _stream(device))
 
 
 class LayerNorm(torch.nn.Module):
@@ -238,24 +262,33 @@ def add_norm(norm: torch.nn.Module, value: torch.Tensor, update: torch.Tensor):
     return total, norm(total)
 
 
-def head_norm_rotary(norm: torch.nn.Module, heads: torch.Tensor, cos: torch.Tensor,
-                     sin: torch.Tensor, dtype: torch.dtype, repeat: int = 1) -> torch.Tensor:
-    """``norm`` of each head of ``[B, S, H, D]``, rotated by ``[1, S, D]``
-    float32 angles and rounded to ``dtype``, every head repeated ``repeat``
-    times; in one pass where the kernels apply."""
+def attention_heads(query_norm: torch.nn.Module, key_norm: torch.nn.Module, q: torch.Tensor,
+                    k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                    dtype: torch.dtype):
+    """The operands of grouped-query attention from ``[B, S, H, D]`` projections:
+    queries and keys through their norms, rotated by ``[1, S, D]`` float32
+    angles and rounded to ``dtype``, key and value heads repeated to the
+    queries' count. One launch where the kernels apply."""
 
-    b, s, h, d = heads.shape
-    if (_unhooked(norm, RMSNorm) and d in (64, 128) and dtype == BF16
-            and _row_kernel(heads, norm.weight)
-            and all(plain_tensor(t) and t.dtype == F32 and t.device == heads.device
+    b, s, h, d = q.shape
+    repeat = h // k.shape[2]
+    if (_unhooked(query_norm, RMSNorm) and _unhooked(key_norm, RMSNorm) and d in (64, 128)
+            and dtype == BF16 and 1 <= repeat and h <= 65536 and k.shape == v.shape
+            and _row_kernel(q, query_norm.weight) and _row_kernel(k, key_norm.weight)
+            and plain_tensor(v) and v.dtype == BF16 and _dense(v)
+            and k.device == q.device == v.device
+            and all(plain_tensor(t) and t.dtype == F32 and t.device == q.device
                     and t.shape == (1, s, d) and _dense(t) and not t.requires_grad
-                    for t in (cos, sin))
-            and h <= 65536 and repeat <= 65536):
-        return HeadNormFn.apply(heads, norm.weight, cos, sin, norm.eps, repeat)
-    value = norm(heads)
-    cos, sin = cos[:, :, None], sin[:, :, None]
-    value = (value.float() * cos + _rotate_half(value.float()) * sin).to(dtype)
-    return value if repeat == 1 else value.repeat_interleave(repeat, dim=2)
+                    for t in (cos, sin))):
+        cfg = ((query_norm.eps, 1), (key_norm.eps, repeat))
+        operands = (q, query_norm.weight, k, key_norm.weight)
+        if repeat == 1:
+            return (*HeadNormFn.apply(cos, sin, cfg, *operands), v)
+        return HeadNormFn.apply(cos, sin, (*cfg, (0.0, repeat)), *operands, v, None)
+    q, k = (rotate(norm(t), cos, sin, dtype) for norm, t in ((query_norm, q), (key_norm, k)))
+    if repeat > 1:
+        k, v = (t.repeat_interleave(repeat, dim=2) for t in (k, v))
+    return q, k, v
 
 
-__all__ = ["LayerNorm", "RMSNorm", "add_norm", "head_norm_rotary"]
+__all__ = ["LayerNorm", "RMSNorm", "add_norm", "attention_heads"]

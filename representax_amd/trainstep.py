@@ -44,7 +44,7 @@ from .adapters import apply_quantized_lora, lora_parameters
 from .components import Linear
 from .config import PrecisionConfig
 from .mlp import gelu_mlp, shared_input_projections, swiglu_mlp
-from .norms import LayerNorm, RMSNorm, add_norm, head_norm_rotary
+from .norms import LayerNorm, RMSNorm, add_norm, attention_heads
 from .precision import (active_compute_views, active_policy, compute_views, precision_context,
                         resolve_precision_policy)
 
@@ -332,14 +332,10 @@ class Qwen3Attention(torch.nn.Module):
     def forward(self, hidden, cos, sin):
         b, s, _ = hidden.shape
         q, k, v = shared_input_projections(hidden, (self.query, self.key, self.value))
-        rep = self.heads // self.kv_heads
-        q = head_norm_rotary(self.query_norm, q.reshape(b, s, self.heads, self.head_dim), cos, sin,
-                             hidden.dtype).transpose(1, 2)
-        k = head_norm_rotary(self.key_norm, k.reshape(b, s, self.kv_heads, self.head_dim), cos,
-                             sin, hidden.dtype, rep).transpose(1, 2)
-        v = v.reshape(b, s, self.kv_heads, self.head_dim).transpose(1, 2)
-        if rep > 1:
-            v = v.repeat_interleave(rep, dim=1)
+        q = q.reshape(b, s, self.heads, self.head_dim)
+        k, v = (t.reshape(b, s, self.kv_heads, self.head_dim) for t in (k, v))
+        q, k, v = attention_heads(self.query_norm, self.key_norm, q, k, v, cos, sin, hidden.dtype)
+        q, k, v = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)
         out = causal_attention(q, k, v, 1.0 / math.sqrt(self.head_dim))
         return self.output(out.transpose(1, 2).reshape(b, s, self.heads * self.head_dim))
 

@@ -9,7 +9,7 @@ import torch
 import torch.nn.functional as F
 
 from representax_amd import norms
-from representax_amd.norms import LayerNorm, RMSNorm, add_norm, head_norm_rotary
+from representax_amd.norms import LayerNorm, RMSNorm, add_norm, attention_heads
 
 DEV = "cuda:0"
 BF16, F64 = torch.bfloat16, torch.float64
@@ -87,21 +87,32 @@ def test_head_norm_with_rotation(b, s, h, d, repeat, weight_dtype):
     angle = torch.randn(1, s, d // 2, generator=g).repeat(1, 1, 2).to(DEV)
     cos, sin = angle.cos(), angle.sin()
     norm = _module("rms", d).to(weight_dtype)
-    y = head_norm_rotary(norm, x, cos, sin, BF16, repeat)
-    assert "HeadNormFn" in type(y.grad_fn).__name__
-    x64 = x.detach().to(F64).requires_grad_(True)
-    n = _want(norm, x64)
-    half = torch.cat((-n[..., d // 2:], n[..., :d // 2]), dim=-1)
-    want = (n * cos.to(F64)[:, :, None] + half * sin.to(F64)[:, :, None])
-    want = want.repeat_interleave(repeat, dim=2)
-    # the normalised value rounds, the rotation keeps its length, the sum rounds
-    assert _rel(y, want) <= 2 * ONE_ROUNDING
+    # queries of h * repeat heads beside keys and values of h heads
+    q = torch.randn(b, s, h * repeat, d, generator=g).to(DEV, BF16).requires_grad_(True)
+    v = torch.randn(b, s, h, d, generator=g).to(DEV, BF16).requires_grad_(True)
+    query_norm = _module("rms", d, seed=1).to(weight_dtype)
+    outs = attention_heads(query_norm, norm, q, x, v, cos, sin, BF16)
+    assert "HeadNormFn" in type(outs[1].grad_fn).__name__
     dy = torch.randn(b, h * repeat, s, d, generator=g).to(DEV, BF16).transpose(1, 2)
-    (dx,) = torch.autograd.grad(y, x, dy, retain_graph=True)
-    (dx64,) = torch.autograd.grad(want, x64, dy.to(F64))
-    assert _rel(dx, dx64) <= ONE_ROUNDING
-    (again,) = torch.autograd.grad(y, x, dy.contiguous())
-    assert torch.equal(dx, again)
+    for n, t, y, rep in ((query_norm, q, outs[0], 1), (norm, x, outs[1], repeat)):
+        t64 = t.detach().to(F64).requires_grad_(True)
+        n64 = _want(n, t64)
+        half = torch.cat((-n64[..., d // 2:], n64[..., :d // 2]), dim=-1)
+        want = (n64 * cos.to(F64)[:, :, None] + half * sin.to(F64)[:, :, None])
+        want = want.repeat_interleave(rep, dim=2)
+        # the normalised value rounds, the rotation keeps its length, the sum rounds
+        assert _rel(y, want) <= 2 * ONE_ROUNDING
+        (dx,) = torch.autograd.grad(y, t, dy, retain_graph=True)
+        (dx64,) = torch.autograd.grad(want, t64, dy.to(F64))
+        assert _rel(dx, dx64) <= ONE_ROUNDING
+        (again,) = torch.autograd.grad(y, t, dy.contiguous(), retain_graph=True)
+        assert torch.equal(dx, again)
+    assert torch.equal(outs[2], v.repeat_interleave(repeat, dim=2))
+    (dv,) = torch.autograd.grad(outs[2], v, dy, retain_graph=True)
+    assert _rel(dv, dy.to(F64).reshape(b, s, h, repeat, d).sum(3)) <= ONE_ROUNDING
+    # all three at once
+    found = torch.autograd.grad(outs, [q, x, v], [dy] * 3)
+    assert torch.equal(found[1], dx) and torch.equal(found[2], dv)
 
 
 @pytest.mark.gpu
@@ -147,9 +158,11 @@ def test_expressions_on_the_cpu():
         norm = _module(kind, 16, "cpu")
         t, y = add_norm(norm, x, r)
         assert torch.equal(t, x + r) and torch.equal(y, norm(x + r))
-    heads = torch.randn(2, 5, 3, 64)
+    q, k, v = (torch.randn(2, 5, n, 64) for n in (6, 3, 3))
     angle = torch.randn(1, 5, 32).repeat(1, 1, 2)
     norm = _module("rms", 64, "cpu")
-    y = head_norm_rotary(norm, heads, angle.cos(), angle.sin(), torch.float32, 2)
-    want = norms.rotate(norm(heads), angle.cos(), angle.sin()).repeat_interleave(2, dim=2)
-    assert torch.equal(y, want)
+    got = attention_heads(norm, norm, q, k, v, angle.cos(), angle.sin(), torch.float32)
+    turned = [norms.rotate(norm(t), angle.cos(), angle.sin()) for t in (q, k)]
+    assert torch.equal(got[0], turned[0])
+    assert torch.equal(got[1], turned[1].repeat_interleave(2, dim=2))
+    assert torch.equal(got[2], v.repeat_interleave(2, dim=2))
