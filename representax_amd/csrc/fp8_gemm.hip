@@ -48,6 +48,37 @@ __device__ __forceinline__ i32x8_t load_frag(const uint8_t* stage, int row, int 
                  (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
 }
 
+// The f8f6f4 MFMA adds its 64 products in fewer bits than float32: against
+// float64 its sums are 4.7e-5 off, whatever their length, where a float32 fma
+// chain over 3500 tokens is 7.4e-8 off. So sums that were float32 chains keep
+// float32 by decoding the codes to bf16 (every fp8 value is one, and so is
+// every product a float32) for four 32x32x16 bf16 MFMAs, which measured 7.3e-8
+// there (1.19e-7 over 8192 tokens, the chain 1.21e-7).
+// Bytes 8 q .. 8 q + 7 of a fragment: MFMA q then sums k = 32 h + 8 q + [0, 8)
+// of both lane halves h, the same k on both operands.
+template <int FMT>
+__device__ __forceinline__ bf16x8_t decode8(i32x8_t f, int q) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  bf16x8_t o;
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    const unsigned v = static_cast<unsigned>(f[2 * q + w]);
+    bf16x2_t lo, hi;
+    if constexpr (FMT == 0) {
+      lo = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 1.0f, false);
+      hi = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 1.0f, true);
+    } else {
+      lo = __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(v, 1.0f, false);
+      hi = __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(v, 1.0f, true);
+    }
+    o[4 * w] = lo[0];
+    o[4 * w + 1] = lo[1];
+    o[4 * w + 2] = hi[0];
+    o[4 * w + 3] = hi[1];
+  }
+  return o;
+}
+
 typedef int i32x2_t __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) i32x2_t lds_i32x2_t;
 
@@ -90,26 +121,33 @@ __device__ __forceinline__ i32x8_t load_frag_krows(const uint8_t* stage, int col
 // Block `bid` of the `nblk` that run this product (a launch may hold other
 // products' blocks too; see k_fp8_gemm_pair).
 //
-// KROWS: both operands are stored with the reduction index as their row, A
-// as [K, M] and B as [K, N] row-major codes (out = A^T B, the weight
-// gradient from the tokens-major codes of the gradient and the input, with
-// no transposed copies). A slice is then 128 rows of 128 code bytes of each
-// operand (128 x 128 tiles only), loaded by the same direct-to-LDS segments
-// and read back through transposing LDS reads (load_frag_krows). Columns
-// past the edge re-read the last 16 bytes of their row (M, N multiples of
-// 16), which only feeds outputs that are never stored. Reduction rows past
-// the end of a ragged K (a token count that is no multiple of 128) are read
-// as zeros: their lanes load from kZeroRow. At 3500 tokens the 768 x 3072
-// weight gradient took 7.7 ms in the one-output-per-thread kernel that
-// served ragged token counts before.
+// kKRows and kKRowsRagged: both operands are stored with the reduction index
+// as their row, A as [K, M] and B as [K, N] row-major codes (out = A^T B, the
+// weight gradient from the tokens-major codes of the gradient and the input,
+// with no transposed copies). A slice is then 128 rows of 128 code bytes of
+// each operand (128 x 128 tiles only), loaded by the same direct-to-LDS
+// segments and read back through transposing LDS reads (load_frag_krows).
+// Columns past the edge re-read the last 16 bytes of their row (M, N multiples
+// of 16), which only feeds outputs that are never stored.
+//
+// kKRowsRagged takes a K (a token count) that is no multiple of 128: reduction
+// rows past its end are read as zeros (their lanes load from kZeroRow), and the
+// sums run on the bf16 MFMAs (decode8), as precise as the one-output-per-thread
+// float32 chain that served these counts before and took 7.9 ms for the 768 x
+// 3072 weight gradient over 3500 tokens. This takes 35.4 us there, bound by the
+// bf16 MFMAs and the decoding before them (the fp8 MFMA took 20.5); with the
+// input gradient in one launch 40.7 against 32.0.
+enum Fp8Layout : int { kRowMajor = 0, kKRows = 1, kKRowsRagged = 2 };
 __device__ const u32x4_t kZeroRow = {0, 0, 0, 0};
 
-template <int BM, int BN, int WM, int WN, int NS, int FA, int FB, bool KROWS = false>
+template <int BM, int BN, int WM, int WN, int NS, int FA, int FB, int LAYOUT = kRowMajor>
 __device__ __forceinline__ void fp8_gemm_block(
     int bid, int nblk, const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int64_t M,
     int64_t N, int64_t K, int64_t k_per_split, const float* __restrict__ s_a,
     const float* __restrict__ s_b, void* __restrict__ out, int out_dtype, int64_t ldc,
     float* __restrict__ partials, int tiles_m, int tiles_n, int band) {
+  constexpr bool KROWS = LAYOUT != kRowMajor;
+  constexpr bool RAGGED = LAYOUT == kKRowsRagged;
   constexpr int NW = WM * WN;
   constexpr int TM = BM / WM;
   constexpr int TN = BN / WN;
@@ -182,11 +220,13 @@ __device__ __forceinline__ void fp8_gemm_block(
   const int kleft = static_cast<int>(kend - kbeg);
   auto dma_one = [&](uint8_t* st, int64_t koff, int i) {
     const int j = wave + i * NW;
-    if constexpr (KROWS) {
+    if constexpr (RAGGED) {
       const int trow = (j < A_SEGS ? 8 * j : 8 * (j - A_SEGS)) + seg_row;
       const uint8_t* p = src[i] + koff * kstep[i];
       p = koff + trow < kleft ? p : reinterpret_cast<const uint8_t*>(&kZeroRow);
       dma_seg(st, p, 0, j);
+    } else if constexpr (KROWS) {
+      dma_seg(st, src[i], koff * kstep[i], j);
     } else {
       dma_seg(st, src[i], koff, j);
     }
@@ -228,8 +268,23 @@ __device__ __forceinline__ void fp8_gemm_block(
   // reads again, which keeps the vmcnt accounting constant (LPW per slice).
   constexpr int NMF = FM * FN;
   constexpr int NFR = FM + FN;
+  // the decoded fragments of a step (RAGGED): block i is the first to use A
+  // fragment i (i < FM) and B fragment i / FM (i % FM == 0)
+  bf16x8_t ad[RAGGED ? FM : 1][4], bd[4];
   auto mma_one = [&](int i, const i32x8_t* af, const i32x8_t* bf) {
-    acc[i / FM][i % FM] = mfma_f8<FB, FA>(bf[i / FM], af[i % FM], acc[i / FM][i % FM]);
+    if constexpr (RAGGED) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (i % FM == 0) bd[q] = decode8<FB>(bf[i / FM], q);
+        if (i < FM) ad[i][q] = decode8<FA>(af[i], q);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        acc[i / FM][i % FM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            bd[q], ad[i % FM][q], acc[i / FM][i % FM], 0, 0, 0);
+    } else {
+      acc[i / FM][i % FM] = mfma_f8<FB, FA>(bf[i / FM], af[i % FM], acc[i / FM][i % FM]);
+    }
   };
   auto frag_one = [&](const uint8_t* st, int kk, int j, i32x8_t* af, i32x8_t* bf) {
     if (j < FM)
@@ -385,13 +440,13 @@ __device__ __forceinline__ void fp8_gemm_block(
   }
 }
 
-template <int BM, int BN, int WM, int WN, int NS, int WPE, int FA, int FB, bool KROWS = false>
+template <int BM, int BN, int WM, int WN, int NS, int WPE, int FA, int FB, int LAYOUT = kRowMajor>
 __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     k_fp8_gemm(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int64_t M, int64_t N,
                int64_t K, int64_t k_per_split, const float* __restrict__ s_a,
                const float* __restrict__ s_b, void* __restrict__ out, int out_dtype, int64_t ldc,
                float* __restrict__ partials, int tiles_m, int tiles_n, int band) {
-  fp8_gemm_block<BM, BN, WM, WN, NS, FA, FB, KROWS>(static_cast<int>(blockIdx.x),
+  fp8_gemm_block<BM, BN, WM, WN, NS, FA, FB, LAYOUT>(static_cast<int>(blockIdx.x),
                                                     static_cast<int>(gridDim.x), A, B, M, N, K,
                                                     k_per_split, s_a, s_b, out, out_dtype, ldc,
                                                     partials, tiles_m, tiles_n, band);
@@ -645,7 +700,7 @@ int fp8_band(int tiles_m, int tiles_n, int64_t blocks, int bm, int bn) {
   return best;
 }
 
-template <int BM, int BN, int WM, int WN, int NS, int WPE, int FA, int FB, bool KROWS = false>
+template <int BM, int BN, int WM, int WN, int NS, int WPE, int FA, int FB, int LAYOUT = kRowMajor>
 hipError_t run_fp8(const uint8_t* a, const uint8_t* b, int64_t m, int64_t n, int64_t k,
                    const Fp8Plan& plan, const float* s_a, const float* s_b, void* out,
                    int out_dtype, int64_t ldc, float* partials, hipStream_t stream) {
@@ -653,7 +708,7 @@ hipError_t run_fp8(const uint8_t* a, const uint8_t* b, int64_t m, int64_t n, int
   static_assert(kLds <= 160 * 1024, "LDS budget");
   const int tiles_m = static_cast<int>(ceil_div(m, BM));
   const int tiles_n = static_cast<int>(ceil_div(n, BN));
-  auto kern = k_fp8_gemm<BM, BN, WM, WN, NS, WPE, FA, FB, KROWS>;
+  auto kern = k_fp8_gemm<BM, BN, WM, WN, NS, WPE, FA, FB, LAYOUT>;
   static std::atomic<unsigned> lds_set{0};
   hipError_t le = ensure_lds_limit(reinterpret_cast<const void*>(kern), kLds, lds_set);
   if (le != hipSuccess) return le;
@@ -701,21 +756,21 @@ Fp8Plan plan_fp8_krows(int64_t m, int64_t n, int64_t k) {
   return plan_for(1, m, n, kslices, nullptr);
 }
 
-template <int FA, int FB>
+template <int FA, int FB, int LAYOUT>
 hipError_t dispatch_fp8_krows(const uint8_t* a, const uint8_t* b, int64_t m, int64_t n, int64_t k,
                               const float* s_a, const float* s_b, void* out, int out_dtype,
                               int64_t ldc, float* partials, hipStream_t stream) {
   const Fp8Plan p = plan_fp8_krows(m, n, k);
   switch (p.cfg) {
     case 1:
-      return run_fp8<128, 128, 2, 2, 2, 2, FA, FB, true>(a, b, m, n, k, p, s_a, s_b, out,
-                                                        out_dtype, ldc, partials, stream);
+      return run_fp8<128, 128, 2, 2, 2, 2, FA, FB, LAYOUT>(a, b, m, n, k, p, s_a, s_b, out,
+                                                          out_dtype, ldc, partials, stream);
     case 6:
-      return run_fp8<128, 128, 2, 2, 4, 1, FA, FB, true>(a, b, m, n, k, p, s_a, s_b, out,
-                                                        out_dtype, ldc, partials, stream);
+      return run_fp8<128, 128, 2, 2, 4, 1, FA, FB, LAYOUT>(a, b, m, n, k, p, s_a, s_b, out,
+                                                          out_dtype, ldc, partials, stream);
     case 9:
-      return run_fp8<128, 128, 2, 2, 3, 2, FA, FB, true>(a, b, m, n, k, p, s_a, s_b, out,
-                                                        out_dtype, ldc, partials, stream);
+      return run_fp8<128, 128, 2, 2, 3, 2, FA, FB, LAYOUT>(a, b, m, n, k, p, s_a, s_b, out,
+                                                          out_dtype, ldc, partials, stream);
     default:
       return hipErrorInvalidValue;
   }
@@ -748,10 +803,10 @@ struct Fp8Cfg {
                        NS = kCfgNS[ID], WPE = kCfgWPE[ID];
 };
 
-template <int ID, int FA, int FB, bool KROWS>
+template <int ID, int FA, int FB, int LAYOUT>
 __device__ __forceinline__ void fp8_part_block(int bid, int nblk, const Fp8Part& p, int out_dtype) {
   using C = Fp8Cfg<ID>;
-  fp8_gemm_block<C::BM, C::BN, C::WM, C::WN, C::NS, FA, FB, KROWS>(
+  fp8_gemm_block<C::BM, C::BN, C::WM, C::WN, C::NS, FA, FB, LAYOUT>(
       bid, nblk, p.a, p.b, p.m, p.n, p.k, p.k_per_split, p.s_a, p.s_b, p.out, out_dtype, p.ldc,
       p.partials, p.tiles_m, p.tiles_n, p.band);
 }
@@ -762,17 +817,17 @@ __device__ __forceinline__ void fp8_part_block(int bid, int nblk, const Fp8Part&
 // and the input), the long reductions over the tokens, which leave most CUs
 // idle on their own (36 tiles x 3 splits for a 768 x 768 weight); the input
 // gradient's tiles, dispatched after them, fill those CUs.
-template <int CW, int CX, int WPE>
+template <int CW, int CX, int WPE, int LAYOUT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     k_fp8_gemm_pair(Fp8Part w, Fp8Part x, int out_dtype) {
   const int b = static_cast<int>(blockIdx.x);
   if (b < w.blocks)
-    fp8_part_block<CW, 1, 0, true>(b, w.blocks, w, out_dtype);
+    fp8_part_block<CW, 1, 0, LAYOUT>(b, w.blocks, w, out_dtype);
   else
-    fp8_part_block<CX, 1, 0, false>(b - w.blocks, x.blocks, x, out_dtype);
+    fp8_part_block<CX, 1, 0, kRowMajor>(b - w.blocks, x.blocks, x, out_dtype);
 }
 
-template <int CW, int CX>
+template <int CW, int CX, int LAYOUT>
 hipError_t run_fp8_pair(Fp8Part w, Fp8Part x, int w_splits, int out_dtype, hipStream_t stream) {
   using W = Fp8Cfg<CW>;
   using X = Fp8Cfg<CX>;
@@ -782,7 +837,7 @@ hipError_t run_fp8_pair(Fp8Part w, Fp8Part x, int w_splits, int out_dtype, hipSt
   constexpr int kLds = kW > kX ? kW : kX;
   constexpr int kWpe = W::WPE < X::WPE ? W::WPE : X::WPE;
   static_assert(kLds <= 160 * 1024, "LDS budget");
-  auto kern = k_fp8_gemm_pair<CW, CX, kWpe>;
+  auto kern = k_fp8_gemm_pair<CW, CX, kWpe, LAYOUT>;
   static std::atomic<unsigned> lds_set{0};
   hipError_t le = ensure_lds_limit(reinterpret_cast<const void*>(kern), kLds, lds_set);
   if (le != hipSuccess) return le;
@@ -880,11 +935,15 @@ hipError_t launch_fp8_backward_pair(const uint8_t* g, const uint8_t* right_codes
   const Fp8Part x = make_part(g, right_codes, m, k, n, px, s_g, s_right, d_left, k, nullptr);
   // d_right^T = ((g^T . left) * s_left) * s_g, the separate launch's order
   const Fp8Part w = make_part(g, left_codes, n, k, m, pw, s_left, s_g, d_right_t, k, split_ws);
+  const bool ragged = m % kBK != 0;
+  const int splits = static_cast<int>(pw.splits);
   hipError_t e;
   if (px.cfg == 4)
-    e = run_fp8_pair<9, 4>(w, x, static_cast<int>(pw.splits), out_dtype, stream);
+    e = ragged ? run_fp8_pair<9, 4, kKRowsRagged>(w, x, splits, out_dtype, stream)
+               : run_fp8_pair<9, 4, kKRows>(w, x, splits, out_dtype, stream);
   else if (px.cfg == 7)
-    e = run_fp8_pair<9, 7>(w, x, static_cast<int>(pw.splits), out_dtype, stream);
+    e = ragged ? run_fp8_pair<9, 7, kKRowsRagged>(w, x, splits, out_dtype, stream)
+               : run_fp8_pair<9, 7, kKRows>(w, x, splits, out_dtype, stream);
   else
     return hipSuccess;
   *launched = e == hipSuccess;
@@ -906,13 +965,19 @@ hipError_t launch_fp8_gemm_krows(const uint8_t* a, int fmt_a, const float* s_a, 
   if (k <= 0 || m % 16 != 0 || n % 16 != 0 ||
       split_ws_floats < fp8_gemm_krows_workspace_floats(m, n, k))
     return hipErrorInvalidValue;
-  if (fmt_a == kE4M3FN && fmt_b == kE4M3FN)
-    return dispatch_fp8_krows<0, 0>(a, b, m, n, k, s_a, s_b, out, out_dtype, ldc, split_ws, stream);
+  // the weight gradient pairs an e5m2 gradient with e4m3 codes, either way round
+  const bool ragged = k % kBK != 0;
   if (fmt_a == kE5M2 && fmt_b == kE4M3FN)
-    return dispatch_fp8_krows<1, 0>(a, b, m, n, k, s_a, s_b, out, out_dtype, ldc, split_ws, stream);
+    return ragged ? dispatch_fp8_krows<1, 0, kKRowsRagged>(a, b, m, n, k, s_a, s_b, out, out_dtype,
+                                                           ldc, split_ws, stream)
+                  : dispatch_fp8_krows<1, 0, kKRows>(a, b, m, n, k, s_a, s_b, out, out_dtype, ldc,
+                                                     split_ws, stream);
   if (fmt_a == kE4M3FN && fmt_b == kE5M2)
-    return dispatch_fp8_krows<0, 1>(a, b, m, n, k, s_a, s_b, out, out_dtype, ldc, split_ws, stream);
-  return dispatch_fp8_krows<1, 1>(a, b, m, n, k, s_a, s_b, out, out_dtype, ldc, split_ws, stream);
+    return ragged ? dispatch_fp8_krows<0, 1, kKRowsRagged>(a, b, m, n, k, s_a, s_b, out, out_dtype,
+                                                           ldc, split_ws, stream)
+                  : dispatch_fp8_krows<0, 1, kKRows>(a, b, m, n, k, s_a, s_b, out, out_dtype, ldc,
+                                                     split_ws, stream);
+  return hipErrorInvalidValue;
 }
 
 }  // namespace rpx

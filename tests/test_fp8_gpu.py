@@ -237,11 +237,12 @@ def _kernel_names(fn):
 
 @pytest.mark.parametrize("m,k,n,paired", [(8192, 768, 768, True), (16384, 768, 768, True),
                                           (8192, 768, 3072, True), (8192, 3072, 768, True),
-                                          (8192, 700, 768, None)])
+                                          (8192, 700, 768, None), (8100, 768, 768, True),
+                                          (8191, 768, 3072, True), (8070, 3072, 768, True)])
 def test_paired_backward_equals_two_launches(m, k, n, paired):
     """The backward's input and weight gradients in one launch (the default
     where both products' plans allow it: the BERT-base linears at 8192
-    tokens) equal the two separate launches bit for bit."""
+    tokens, and ragged counts just below) equal the two separate launches bit for bit."""
 
     x, w, gy = _fp8_case(m, k, n, seed=m + 5 * k + n)
     _, scales, codes = ops.fp8_linear_forward(to_dev_bf16(x), to_dev_bf16(w).t(),

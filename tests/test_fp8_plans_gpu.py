@@ -33,7 +33,7 @@ import torch
 import representax_amd as rx
 from oracle import fp8 as ofp8
 from oracle import int4 as oint4
-from oracle.codecs import E4M3FN, E5M2, bf16_bits_to_f32, bf16_round
+from oracle.codecs import E4M3FN, E5M2, bf16_bits_to_f32, bf16_round, fp8_decode
 from representax_amd import ops
 from tests.helpers import (assert_bf16_close, bf16_values,
                            from_dev, rel_l2, rng, to_dev, to_dev_bf16)
@@ -166,7 +166,7 @@ def test_fp8_step_calls_full_size_match_oracle(call):
     assert torch.equal(b16.view(torch.int16), f32.to(torch.bfloat16).view(torch.int16))
 
 
-def _weight_grad_krows(qx, s_x, qg, s_g, right_t):
+def _weight_grad_krows(qx, s_x, qg, s_g, right_t, dtype=torch.bfloat16):
     """d_right of the fp8 linear backward through the K-row kernel (the
     tokens-major codes of the input and the gradient as they are): [N, K]
     when right_t, else [K, N]."""
@@ -176,7 +176,7 @@ def _weight_grad_krows(qx, s_x, qg, s_g, right_t):
     dummy = torch.zeros((k, n), dtype=torch.uint8, device="cuda")
     _, d_right = ops.fp8_linear_backward_gemms(
         qg, torch.tensor([s_g], device="cuda"), qx, torch.tensor([s_x], device="cuda"), dummy,
-        torch.tensor([1.0], device="cuda"), k=k, dtype=torch.bfloat16, right_transposed=right_t,
+        torch.tensor([1.0], device="cuda"), k=k, dtype=dtype, right_transposed=right_t,
         need_left=False)
     return d_right.t() if right_t else d_right
 
@@ -257,6 +257,50 @@ def test_weight_gradient_krows_ragged_tokens(m, right_t):
         torch.cuda.synchronize()
         assert_bf16_close(from_dev(got), bf16_round(want), tol=FP8_TOL, min_equal=None,
                           what=f"{m}x{k}x{n} right_t={right_t} splits={splits}")
+
+
+@pytest.mark.parametrize("right_t", [True, False])
+@pytest.mark.parametrize("m", [1, 127, 129, 1295, 3500])
+def test_weight_gradient_ragged_tokens_sums_in_float32(m, right_t):
+    """Over a token count that is no multiple of 128 the sums are float32 (the
+    fp8 MFMA's are not: 4.7e-5 off here). Each of m additions rounds by at most
+    2^-24 of a partial sum that grows as a random walk, 2^-24 sqrt(m / 6) of
+    the result in the root mean square, and the two scales round twice more;
+    twice that is allowed. bf16 outputs are the float32 ones, rounded."""
+
+    k, n = 208, 400
+    g = rng(5000 + m)
+    qx, s_x = _quantized(g, (m, k), E4M3FN, outliers=True)
+    qg, s_g = _quantized(g, (m, n), E5M2)
+    if right_t:
+        want = ofp8.scaled_dot_codes(np.ascontiguousarray(qg.T), s_x, E5M2, qx, s_g, E4M3FN)
+    else:
+        want = ofp8.scaled_dot_codes(np.ascontiguousarray(qx.T), s_x, E4M3FN, qg, s_g, E5M2)
+    qxd, qgd = to_dev(qx), to_dev(qg)
+    for splits in (0, 1, 3):
+        if splits > -(-m // 128):
+            continue
+        with ops.tuning(fp8_splits=splits):
+            f32 = _weight_grad_krows(qxd, s_x, qgd, s_g, right_t, torch.float32)
+            b16 = _weight_grad_krows(qxd, s_x, qgd, s_g, right_t)
+        torch.cuda.synchronize()
+        assert rel_l2(from_dev(f32), want) <= 2.0 * 2.0 ** -24 * (np.sqrt(m / 6.0) + 2.0), splits
+        assert torch.equal(b16.view(torch.int16), f32.to(torch.bfloat16).view(torch.int16))
+
+
+def test_weight_gradient_of_one_token_takes_every_code():
+    """One token: every output is one product, so all 256 codes of either
+    format (subnormals, infinities and NaN among them) come out as decoded."""
+
+    codes = np.arange(256, dtype=np.uint8)[None]
+    ones = {E4M3FN: np.full((1, 16), 0x38, np.uint8), E5M2: np.full((1, 16), 0x3C, np.uint8)}
+    one = np.float32(1.0)
+    got = _weight_grad_krows(to_dev(codes), one, to_dev(ones[E5M2]), one, False, torch.float32)
+    want = np.repeat(fp8_decode(codes, E4M3FN).T, 16, axis=1)
+    np.testing.assert_array_equal(from_dev(got), want)
+    got = _weight_grad_krows(to_dev(ones[E4M3FN]), one, to_dev(codes), one, True, torch.float32)
+    want = np.repeat(fp8_decode(codes, E5M2).T, 16, axis=1)
+    np.testing.assert_array_equal(from_dev(got), want)
 
 
 @pytest.mark.parametrize("m,k,n", [(200, 40, 30), (256, 24, 136), (384, 128, 100)])
