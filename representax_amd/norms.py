@@ -200,8 +200,11 @@ class HeadNormFn(torch.autograd.Function):
 
 
 def _head_norm(cos, sin, cfg, xs, weights, grads, outs) -> None:
-    device = _on_device(cos, sin, *xs, *weights)
     b, s, _, d = xs[0].shape
+    if any(x.shape != (b, s, x.shape[2], d) for x in xs):
+        raise ValueError(f"parts of one launch have the same tokens and head width, got "
+                         f"{[tuple(x.shape) for x in xs]}")
+    device = _on_device(cos, sin, *xs, *weights)
     parts = (nat.HeadPart * len(xs))()
     for i, (x, w, (eps, repeat)) in enumerate(zip(xs, weights, cfg)):
         part = parts[i]
@@ -273,7 +276,8 @@ def attention_heads(query_norm: torch.nn.Module, key_norm: torch.nn.Module, q: t
     b, s, h, d = q.shape
     repeat = h // k.shape[2]
     if (_unhooked(query_norm, RMSNorm) and _unhooked(key_norm, RMSNorm) and d in (64, 128)
-            and dtype == BF16 and 1 <= repeat and h <= 65536 and k.shape == v.shape
+            and dtype == BF16 and h <= 65536 and repeat * k.shape[2] == h
+            and k.shape == v.shape == (b, s, k.shape[2], d)  # the launch reads b * s tokens of each
             and _row_kernel(q, query_norm.weight) and _row_kernel(k, key_norm.weight)
             and plain_tensor(v) and v.dtype == BF16 and _dense(v)
             and k.device == q.device == v.device

@@ -166,3 +166,33 @@ def test_expressions_on_the_cpu():
     assert torch.equal(got[0], turned[0])
     assert torch.equal(got[1], turned[1].repeat_interleave(2, dim=2))
     assert torch.equal(got[2], v.repeat_interleave(2, dim=2))
+
+
+@pytest.mark.parametrize("kv,route", [((2, 5, 2, 64), True), ((2, 5, 4, 64), True),
+                                      ((2, 3, 2, 64), False), ((1, 5, 2, 64), False),
+                                      ((2, 5, 2, 128), False), ((2, 5, 3, 64), False)])
+def test_attention_heads_launches_only_over_matching_tokens(monkeypatch, kv, route):
+    """The launch reads the queries' token count of every part: keys and values
+    of other tokens, batches or head widths (or head counts that do not divide
+    the queries') stay on the torch expressions, which raise or broadcast."""
+
+    taken = []
+    monkeypatch.setattr(norms, "plain_tensor", lambda t: True)
+    monkeypatch.setattr(norms, "_row_kernel", lambda *a: True)
+    monkeypatch.setattr(RMSNorm, "forward", lambda m, t: norms.rms_norm(t, m.weight, m.eps))
+    monkeypatch.setattr(norms.HeadNormFn, "apply", lambda *a: taken.append(a) or (q, k, v))
+    q, k, v = (torch.randn(s).to(BF16) for s in ((2, 5, 4, 64), kv, kv))
+    norm, key_norm = _module("rms", 64, "cpu"), _module("rms", kv[3], "cpu")
+    angle = torch.randn(1, 5, 32).repeat(1, 1, 2)
+    call = (norm, key_norm, q, k, v, angle.cos(), angle.sin(), BF16)
+    if kv[1] != 5 or kv[3] != 64:
+        with pytest.raises(RuntimeError):  # the rotation meets angles of other tokens
+            attention_heads(*call)
+    else:
+        outs = attention_heads(*call)
+        if kv[0] == 1:  # a batch that attention broadcasts
+            assert outs[1].shape == outs[2].shape == (1, 5, 4, 64)
+    assert bool(taken) == route
+    if not route and kv[2] == 2:
+        with pytest.raises(ValueError, match="same tokens"):
+            norms._head_norm(angle, angle, ((1e-6, 1),) * 2, (q, k), (norm.weight,) * 2, None, None)
