@@ -218,11 +218,13 @@ int rpx_int4lora_forward_multi(const void* x, int dtype, int64_t m, int64_t k, i
  * harnesses that forbid hipMalloc); no counterpart in the reference. Scratch
  * (the skinny-M kernels' split partials) comes from a static device buffer of
  * RPX_STATIC_SCRATCH_BYTES per GPU that the library holds until the process
- * ends; the entry point itself calls no allocator. A call that needs more
- * scratch than that (rpx_int4lora_forward_workspace() above the limit, e.g.
- * the generic path of a large unaligned shape) is rejected with
- * RPX_ERR_INVALID before anything is launched. Every call on a GPU shares that
- * GPU's buffer: calls that overlap on one GPU (different streams) race. */
+ * ends; the entry point itself calls no allocator. A call that cannot do
+ * without more scratch than that (e.g. the generic path of a large unaligned
+ * shape) is rejected with RPX_ERR_INVALID before anything is launched; the
+ * bf16 weight copy that rpx_int4lora_forward_workspace() counts for large
+ * calls is optional and not taken here. Every call on a GPU shares that GPU's
+ * buffer: calls that use it (M <= 64, and shapes off the MFMA path) race where
+ * they overlap on one GPU (different streams); the others use no scratch. */
 #define RPX_STATIC_SCRATCH_BYTES (16u << 20)
 int rpx_int4lora_forward_static(const void* x, int dtype, int64_t m, int64_t k,
                                 const uint8_t* packed, const uint16_t* scale_bits, int64_t n,

@@ -759,8 +759,9 @@ int rpx_int4lora_forward_static(const void* x, int dtype, int64_t m, int64_t k,
                                 int64_t group_size, const uint16_t* bias_bits, const void* lora_a,
                                 const void* lora_b, int64_t rank, float scaling, void* y, void* h,
                                 void* stream) {
-  // the wide GEMM's W_b copy is optional: a call that it does not fit takes
-  // the fused GEMM
+  // what the call cannot do without: the wide GEMM's W_b copy is not taken
+  // from the buffer that every call shares, so large calls run the fused GEMM
+  // and touch no scratch
   int64_t ng = 1, g = k;
   if (group_size > 0 && group_size != k && k % group_size == 0) {
     ng = k / group_size;
@@ -778,8 +779,7 @@ int rpx_int4lora_forward_static(const void* x, int dtype, int64_t m, int64_t k,
   void* ws = nullptr;
   if (m > 0 && n > 0) RPX_TRY(static_scratch(&ws));
   return int4lora_forward_impl(x, dtype, m, k, packed, scale_bits, n, group_size, bias_bits, lora_a,
-                               lora_b, rank, scaling, y, h, ws, kStaticScratchBytes, stream,
-                               ActIO{});
+                               lora_b, rank, scaling, y, h, ws, need, stream, ActIO{});
 }
 
 int rpx_int4lora_forward_act(const void* x, int dtype, int64_t m, int64_t k, const uint8_t* packed,

@@ -111,3 +111,12 @@ def assert_bf16_close(got: np.ndarray, want: np.ndarray, tol: float = BF16_REL_T
         eq = float(np.mean(same))
         allowed = max(1, int(np.floor((1.0 - min_equal) * same.size)))
         assert eq >= min_equal or int(same.size - same.sum()) <= allowed, (what, eq)
+
+
+def kernel_names(fn):
+    """``fn()`` and the names of the device kernels that it ran."""
+
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        out = fn()
+        torch.cuda.synchronize()
+    return out, [e.key for e in prof.key_averages()]

@@ -13,7 +13,7 @@ from oracle import int4 as oint4
 from oracle.codecs import f32_to_bf16_bits
 from representax_amd import _native as nat
 from representax_amd import ops
-from tests.helpers import bf16_values, rng, to_dev, to_dev_bf16
+from tests.helpers import bf16_values, kernel_names, rng, to_dev, to_dev_bf16
 
 pytestmark = pytest.mark.gpu
 
@@ -65,6 +65,24 @@ def test_static_forward_equals_workspace_forward(m1, m2, k, n, r, group):
                                       scaling=2.0, group_size=group, bias_bits=lin["bias"])
         torch.cuda.synchronize()
         assert torch.equal(ys, yw) and torch.equal(hs, hw), m
+
+
+def test_static_forward_of_a_large_call_uses_no_scratch():
+    """A call whose optional bf16 weight copy would fit the static buffer keeps
+    the GEMM without it: large calls on several streams share nothing."""
+
+    m, k, n, r = 16384, 768, 3072, 16
+    lin = _linear(n, k, r, 64, seed=11)
+    x = to_dev_bf16(bf16_values(rng(12).standard_normal((m, k))))
+    copy = nat.query("rpx_int4lora_forward_workspace", m, n, k, 64, r, nat.DTYPE_BF16)
+    assert 2 * n * k <= copy <= STATIC_BYTES
+    (yw, hw), names = kernel_names(lambda: ops.int4lora_forward(
+        x, lin["packed"], lin["scales"], lin["a"], lin["b"], scaling=2.0, group_size=64,
+        bias_bits=lin["bias"]))
+    assert any("k_gemm_wide" in name for name in names)
+    (ys, hs), names = kernel_names(lambda: _static_forward(lin, x))
+    assert names and not any("k_gemm_wide" in name or "dequant" in name for name in names)
+    assert torch.equal(ys, yw) and torch.equal(hs, hw)
 
 
 def test_static_forward_rejects_calls_beyond_its_scratch():
