@@ -70,11 +70,12 @@ def _frozen(size: int, device, *weights: torch.Tensor) -> bool:
 
 
 def _row_kernel(value: torch.Tensor, *weights: torch.Tensor) -> bool:
+    if not eager_calls():
+        return False
     size = value.shape[-1] if value.dim() else 0
     return (plain_tensor(value) and value.dtype == BF16 and 8 <= size <= _MAX_SIZE
             and size % 8 == 0 and 0 < value.numel() and value.numel() // size <= 1 << 31 and _dense(value)
-            and _frozen(size, value.device, *weights) and eager_calls()
-            and not torch.is_autocast_enabled("cuda"))
+            and _frozen(size, value.device, *weights) and not torch.is_autocast_enabled("cuda"))
 
 
 def _unhooked(module: torch.nn.Module, cls: type) -> bool:
@@ -254,7 +255,7 @@ def add_norm(norm: torch.nn.Module, value: torch.Tensor, update: torch.Tensor):
     where the kernels apply."""
 
     kind = {LayerNorm: nat.NORM_LAYER, RMSNorm: nat.NORM_RMS}.get(type(norm))
-    if kind is not None and _unhooked(norm, type(norm)):
+    if kind is not None and eager_calls() and _unhooked(norm, type(norm)):
         bias = norm.bias if kind == nat.NORM_LAYER else None
         weights = (norm.weight,) if bias is None else (norm.weight, bias)
         if (_row_kernel(value, *weights) and plain_tensor(update) and update.dtype == BF16
@@ -275,7 +276,8 @@ def attention_heads(query_norm: torch.nn.Module, key_norm: torch.nn.Module, q: t
 
     b, s, h, d = q.shape
     repeat = h // k.shape[2]
-    if (_unhooked(query_norm, RMSNorm) and _unhooked(key_norm, RMSNorm) and d in (64, 128)
+    if (eager_calls() and _unhooked(query_norm, RMSNorm) and _unhooked(key_norm, RMSNorm)
+            and d in (64, 128)
             and dtype == BF16 and h <= 65536 and repeat * k.shape[2] == h
             and k.shape == v.shape == (b, s, k.shape[2], d)  # the launch reads b * s tokens of each
             and _row_kernel(q, query_norm.weight) and _row_kernel(k, key_norm.weight)

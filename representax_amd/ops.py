@@ -692,18 +692,24 @@ CAST_MANY = 16  # tensors of one launch
 
 
 def plain_tensor(t: torch.Tensor) -> bool:
-    """An ordinary device tensor: no subclass, no function-transform wrapper."""
+    """An ordinary device tensor: no subclass, no function-transform wrapper,
+    no batched gradient (those have no storage of their own)."""
 
     return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
-            and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and torch._C._has_storage(t))
 
 
 def eager_calls() -> bool:
     """Nothing watches or rewrites torch operations: one kernel may stand for
-    several of them."""
+    several of them. Asked before anything about a tensor: a compiler's trace
+    ends at the first question and meets no call that it cannot trace. Under a
+    function transform an autograd function is refused also where its tensors
+    are only closed over."""
 
     return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
                 or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch._C._are_functorch_transforms_active()
                 or torch.autograd.forward_ad._current_level >= 0)
 
 
@@ -712,10 +718,10 @@ def cast_many(tensors, dtype: torch.dtype) -> list[torch.Tensor]:
     dense tensors of one device (no autograd)."""
 
     device = tensors[0].device
-    if not (dtype == BF16 and 1 < len(tensors) <= CAST_MANY
+    if not (dtype == BF16 and 1 < len(tensors) <= CAST_MANY and eager_calls()
             and all(t.dtype == F32 and plain_tensor(t) and t.device == device
                     and t.is_contiguous() and t.numel() and t.data_ptr() % 16 == 0
-                    for t in tensors) and eager_calls()):
+                    for t in tensors)):
         return [t.to(dtype) for t in tensors]
     out = [torch.empty_like(t, dtype=BF16) for t in tensors]
     count = len(tensors)

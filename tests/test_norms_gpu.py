@@ -8,7 +8,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from representax_amd import norms
+from representax_amd import norms, ops
 from representax_amd.norms import LayerNorm, RMSNorm, add_norm, attention_heads
 
 DEV = "cuda:0"
@@ -196,3 +196,62 @@ def test_attention_heads_launches_only_over_matching_tokens(monkeypatch, kv, rou
     if not route and kv[2] == 2:
         with pytest.raises(ValueError, match="same tokens"):
             norms._head_norm(angle, angle, ((1e-6, 1),) * 2, (q, k), (norm.weight,) * 2, None, None)
+
+
+def _cpu_routes(monkeypatch):
+    """The routes' conditions on CPU tensors: everything but their device."""
+
+    def plain(t):
+        return (type(t) in (torch.Tensor, torch.nn.Parameter)
+                and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+                and torch._C._has_storage(t))
+
+    monkeypatch.setattr(norms, "plain_tensor", plain)
+
+
+def test_transforms_and_compilers_keep_the_expressions(monkeypatch):
+    """Inside a function transform a tensor that is closed over is no wrapper,
+    but an autograd function is refused all the same; a compiler cannot trace
+    the conditions. Both get the torch expressions."""
+
+    _cpu_routes(monkeypatch)
+    x, r = (torch.randn(4, 16).to(BF16) for _ in range(2))
+    norm, bias = _module("rms", 16, "cpu"), _module("layer", 16, "cpu")
+    assert norms._row_kernel(x, norm.weight)
+    seen = []
+
+    def closed_over(value):
+        seen.append(norms._row_kernel(x, norm.weight))
+        return add_norm(norm, x, r)[1].float().sum() * value
+
+    torch.func.vmap(closed_over)(torch.ones(3))
+    torch.func.grad(closed_over)(torch.ones(()))
+    torch.func.jvp(closed_over, (torch.ones(()),), (torch.ones(()),))
+    assert seen == [False] * 3
+    for module in (norm, bias):
+        compiled = torch.compile(module, fullgraph=True, backend="eager")
+        assert torch.equal(compiled(x), norms._expression(
+            int(module is norm), x, module.weight, getattr(module, "bias", None), module.eps))
+    compiled = torch.compile(lambda v: add_norm(norm, v, r), fullgraph=True, backend="eager")
+    assert torch.equal(compiled(x)[1], norms.rms_norm(x + r, norm.weight, norm.eps))
+    angle = torch.randn(1, 5, 32).repeat(1, 1, 2)
+    q, k, v = (torch.randn(2, 5, n, 64).to(BF16) for n in (4, 2, 2))
+    head = _module("rms", 64, "cpu")
+    compiled = torch.compile(lambda *t: attention_heads(head, head, *t, angle.cos(), angle.sin(), BF16),
+                             fullgraph=True, backend="eager")
+    assert torch.equal(compiled(q, k, v)[2], v.repeat_interleave(2, dim=2))
+
+
+@pytest.mark.gpu
+def test_transforms_and_compilers_on_the_device():
+    x, r = (torch.randn(4, 64, device=DEV).to(BF16) for _ in range(2))
+    norm = _module("rms", 64)
+    want = norms.rms_norm(x + r, norm.weight, norm.eps)
+    rows = torch.func.vmap(lambda c: add_norm(norm, x, r)[1] * c)(torch.ones(2, device=DEV, dtype=BF16))
+    assert torch.equal(rows[1], want)
+    compiled = torch.compile(lambda v: add_norm(norm, v, r)[1], fullgraph=True, backend="eager")
+    assert torch.equal(compiled(x), want)
+    masters = [torch.randn(8, 64, device=DEV) for _ in range(2)]
+    views = torch.func.vmap(lambda c: ops.cast_many(masters, BF16)[0] * c)(
+        torch.ones(2, device=DEV, dtype=BF16))
+    assert torch.equal(views[0], masters[0].to(BF16))
