@@ -108,6 +108,15 @@ def _expression(kind: int, value, weight, bias, eps):
     return layer_norm(value, weight, bias, eps)
 
 
+def _kernel_gradients(*grads) -> bool:
+    """The backward kernels take these gradients. Not where the gradient is
+    itself differentiated (create_graph), batched (is_grads_batched) or traced:
+    there the expressions are differentiated instead."""
+
+    return (not torch.is_grad_enabled() and eager_calls()
+            and all(g is None or plain_tensor(g) for g in grads))
+
+
 def _gradient(ctx, dy, d_total):
     """The gradient of the normalised row for the gradients of the norm and
     (or None) of the row's other use."""
@@ -115,9 +124,11 @@ def _gradient(ctx, dy, d_total):
     value, weight, bias = ctx.saved_tensors
     if dy is None:
         return d_total
-    if torch.is_grad_enabled():  # create_graph: the gradient is differentiated again
-        y = _expression(ctx.kind, value, weight, bias, ctx.eps)
-        dx, = torch.autograd.grad(y, value, dy, create_graph=True)
+    if not _kernel_gradients(dy, d_total):
+        again = torch.is_grad_enabled()
+        with torch.enable_grad():
+            y = _expression(ctx.kind, value, weight, bias, ctx.eps)
+        dx, = torch.autograd.grad(y, value, dy, create_graph=again)
         return dx if d_total is None else dx + d_total
     device = _on_device(value, dy)
     size = value.shape[-1]
@@ -185,12 +196,14 @@ class HeadNormFn(torch.autograd.Function):
     def backward(ctx, *grads):
         cos, sin, *operands = ctx.saved_tensors
         xs, weights = operands[::2], operands[1::2]
-        if torch.is_grad_enabled():  # create_graph: the gradient is differentiated again
+        if not _kernel_gradients(*grads):
+            again = torch.is_grad_enabled()
             found = []
             for x, w, g, (eps, repeat) in zip(xs, weights, grads, ctx.cfg):
-                y = x if w is None else rotate(rms_norm(x, w, eps), cos, sin)
-                y = y.repeat_interleave(repeat, dim=2)
-                found += [torch.autograd.grad(y, x, g, create_graph=True)[0]
+                with torch.enable_grad():
+                    y = x if w is None else rotate(rms_norm(x, w, eps), cos, sin)
+                    y = y.repeat_interleave(repeat, dim=2)
+                found += [torch.autograd.grad(y, x, g, create_graph=again)[0]
                           if x.requires_grad else None, None]
             return (None, None, None, *found)
         grads = [g if g.stride(3) == 1 and not any(n % 8 for n in g.stride()[:3])

@@ -255,3 +255,54 @@ def test_transforms_and_compilers_on_the_device():
     views = torch.func.vmap(lambda c: ops.cast_many(masters, BF16)[0] * c)(
         torch.ones(2, device=DEV, dtype=BF16))
     assert torch.equal(views[0], masters[0].to(BF16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_batched_gradients(create_graph):
+    """Several gradients at once (is_grads_batched, vectorized Jacobians) have
+    no storage for a kernel to read; the expressions are differentiated."""
+
+    x, r = (torch.randn(3, 5, 64, device=DEV).to(BF16).requires_grad_(True) for _ in range(2))
+    for kind in ("layer", "rms"):
+        norm = _module(kind, 64)
+        dy = torch.randn(4, 3, 5, 64, device=DEV).to(BF16)
+        for y, leaves in ((norm(x), [x]), (add_norm(norm, x, r)[1], [x, r])):
+            assert "NormFn" in type(y.grad_fn).__name__
+            one = [torch.autograd.grad(y, leaves, g, retain_graph=True) for g in dy]
+            all_ = torch.autograd.grad(y, leaves, dy, is_grads_batched=True, retain_graph=True,
+                                       create_graph=create_graph)
+            for i, got in enumerate(all_):
+                assert got.shape == dy.shape
+                for j in range(4):  # both within one rounding of float64
+                    assert _rel(got[j], one[j][i].to(F64)) <= 2 * ONE_ROUNDING
+    q, k, v = (torch.randn(2, 5, n, 64, device=DEV).to(BF16).requires_grad_(True) for n in (4, 2, 2))
+    angle = torch.randn(1, 5, 32, device=DEV).repeat(1, 1, 2)
+    norm = _module("rms", 64)
+    outs = attention_heads(norm, norm, q, k, v, angle.cos(), angle.sin(), BF16)
+    assert "HeadNormFn" in type(outs[1].grad_fn).__name__
+    dy = torch.randn(3, 2, 5, 4, 64, device=DEV).to(BF16)
+    for y, t in zip(outs, (q, k, v)):
+        (got,) = torch.autograd.grad(y, t, dy, is_grads_batched=True, retain_graph=True,
+                                     create_graph=create_graph)
+        for j in range(3):
+            (one,) = torch.autograd.grad(y, t, dy[j], retain_graph=True)
+            # the expression rounds the rotated gradient, the repeated heads'
+            # sum and the result, the kernel the result
+            assert _rel(got[j], one.to(F64)) <= 4 * ONE_ROUNDING
+
+
+def test_batched_gradients_reach_no_kernel(monkeypatch):
+    _cpu_routes(monkeypatch)
+    monkeypatch.setattr(norms, "_forward", lambda x, r, w, b, kind, eps: (
+        None, norms._expression(kind, x, w, b, eps)))
+    x = torch.randn(4, 16, dtype=torch.float32).to(BF16).requires_grad_(True)
+    norm = _module("rms", 16, "cpu")
+    y = norms.NormFn.apply(x, norm.weight, None, norms.nat.NORM_RMS, norm.eps)
+    dy = torch.randn(5, 4, 16).to(BF16)
+    with pytest.raises(RuntimeError, match="ROCm devices only"):  # one gradient: the kernel's
+        torch.autograd.grad(y, x, dy[0], retain_graph=True)
+    (got,) = torch.autograd.grad(y, x, dy, is_grads_batched=True)
+    for i in range(5):
+        (want,) = torch.autograd.grad(norms.rms_norm(x, norm.weight, norm.eps), x, dy[i])
+        assert _rel(got[i], want.to(F64)) <= 2 * ONE_ROUNDING
