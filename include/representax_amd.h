@@ -530,7 +530,8 @@ int rpx_mnr_backward(const float* grad_loss, const void* saved, size_t saved_byt
 #define RPX_NORM_RMS 1
 
 /* y = norm(t) over rows [rows, size], t = x, or bf16(x + residual) when
- * residual is given (then `sum` receives t). LayerNorm takes its weight and
+ * residual is given. `sum` receives t; it is required with a residual and may
+ * be NULL without. LayerNorm takes its weight and
  * bias rounded to bf16. Requires size a multiple of 8, at most 4096. */
 int rpx_norm_forward(const void* x, const void* residual, const void* weight, const void* bias,
                      int weight_dtype, int64_t rows, int64_t size, float eps, int kind, void* sum,

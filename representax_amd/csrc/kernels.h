@@ -296,8 +296,8 @@ struct NormArgs {
   int64_t rows;
   int size;  // a multiple of 8, at most kNormMaxSize
   float eps;
-  uint16_t* sum;  // bf16(x + residual), written when there is a residual; backward: the
-                  // normalised row, read
+  uint16_t* sum;  // bf16(x + residual) or x, written unless nullptr; backward: the normalised
+                  // row, read
   uint16_t* y;    // backward: the gradient of the row
 };
 

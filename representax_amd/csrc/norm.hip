@@ -96,8 +96,8 @@ __device__ __forceinline__ void row_stats(const float (&v)[C][8], int lane, int 
   *rstd = rsqrtf(row_sum<L>(s) / static_cast<float>(size) + eps);
 }
 
-// y = norm(t), t = x or bf16(x + r) (then also written): L lanes a row, C
-// chunks of 8 elements a lane.
+// y = norm(t), t = x or bf16(x + r), also written where there is a `sum` for
+// it: L lanes a row, C chunks of 8 elements a lane.
 template <int KIND, bool ADD, int L, int C>
 __global__ void __launch_bounds__(kThreads)
     k_norm_fwd(const uint16_t* __restrict__ x, const uint16_t* __restrict__ r,
@@ -114,16 +114,17 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[c][i] = 0.0f;
     if (e >= size) continue;
-    load8(x + base + e, v[c]);
+    u32x4_t t = *reinterpret_cast<const u32x4_t*>(x + base + e);
+    unpack8(t, v[c]);
     if constexpr (ADD) {
       float a[8];
       load8(r + base + e, a);
 #pragma unroll
       for (int i = 0; i < 8; ++i) a[i] += v[c][i];
-      const u32x4_t t = pack8(a);
-      *reinterpret_cast<u32x4_t*>(sum + base + e) = t;
+      t = pack8(a);
       unpack8(t, v[c]);
     }
+    if (ADD || sum != nullptr) *reinterpret_cast<u32x4_t*>(sum + base + e) = t;
   }
   // the weights' loads are in flight while the statistics are summed
   float g[C][8], h[KIND == kNormLayer ? C : 1][8];

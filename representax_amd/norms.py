@@ -7,7 +7,8 @@ after it (src/representax/models/qwen3_vl/text.py:30-61).
 The kernels take bf16 device values with frozen weights; everything else
 (float32, trainable norm weights, autocast, function transforms, tracing,
 other widths and layouts) runs the torch expressions, which also define the
-values: both round to bf16 at the same places.
+values: both round to bf16 at the same places. The frozen weights are saved for
+the backward as they are, so they do not change between a call and its backward.
 """
 
 from __future__ import annotations
@@ -91,11 +92,13 @@ def _unhooked(module: torch.nn.Module, cls: type) -> bool:
 # ---------------------------------------------------------------------------
 # the fused calls
 # ---------------------------------------------------------------------------
-def _forward(x, residual, weight, bias, kind: int, eps: float):
+def _forward(x, residual, weight, bias, kind: int, eps: float, keep: bool = False):
+    """``(t, norm(t))``, t = x + residual, or a copy of x with ``keep`` (else None)."""
+
     device = _on_device(x, residual, weight, bias)
     size = x.shape[-1]
     y = torch.empty_like(x)
-    total = None if residual is None else torch.empty_like(x)
+    total = torch.empty_like(x) if keep or residual is not None else None
     nat.call("rpx_norm_forward", _ptr(x), _ptr(residual), _ptr(weight), _ptr(bias),
              _dtype_code(weight.dtype), x.numel() // size, size, float(eps), kind, _ptr(total),
              _ptr(y), _stream(device))
@@ -156,20 +159,21 @@ class NormFn(torch.autograd.Function):
 
 
 class AddNormFn(torch.autograd.Function):
-    """``t = x + residual`` and its norm, with frozen weights: ``(t, norm(t))``."""
+    """``t = x + residual`` (or, without a residual, a copy of x) and its norm,
+    with frozen weights: ``(t, norm(t))``. The backward reads t."""
 
     @staticmethod
     def forward(ctx, x, residual, weight, bias, kind, eps):
         ctx.set_materialize_grads(False)
-        total, y = _forward(x, residual, weight, bias, kind, eps)
+        total, y = _forward(x, residual, weight, bias, kind, eps, keep=True)
         ctx.save_for_backward(total, weight, bias)
-        ctx.kind, ctx.eps = kind, eps
+        ctx.kind, ctx.eps, ctx.added = kind, eps, residual is not None
         return total, y
 
     @staticmethod
     def backward(ctx, d_total, dy):
         dx = _gradient(ctx, dy, d_total)
-        return dx, dx, None, None, None, None
+        return dx, dx if ctx.added else None, None, None, None, None
 
 
 class HeadNormFn(torch.autograd.Function):
@@ -186,7 +190,11 @@ class HeadNormFn(torch.autograd.Function):
         xs, weights = operands[::2], operands[1::2]
         b, s, _, d = xs[0].shape
         ctx.cfg = cfg
-        ctx.save_for_backward(cos, sin, *operands)
+        # a part that is only repeated: its gradient does not depend on it
+        kept = [t for x, w in zip(xs, weights) if w is not None for t in (x, w)]
+        ctx.normed = [w is not None for w in weights]
+        ctx.heads = [x.shape[2] for x in xs]
+        ctx.save_for_backward(cos, sin, *kept)
         outs = [torch.empty((b, s, x.shape[2] * repeat, d), dtype=BF16, device=x.device)
                 for x, (_, repeat) in zip(xs, cfg)]
         _head_norm(cos, sin, cfg, xs, weights, None, outs)
@@ -194,22 +202,29 @@ class HeadNormFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, *grads):
-        cos, sin, *operands = ctx.saved_tensors
-        xs, weights = operands[::2], operands[1::2]
+        cos, sin, *kept = ctx.saved_tensors
+        saved = iter(kept)
+        pairs = [(next(saved), next(saved)) if normed else (None, None) for normed in ctx.normed]
         if not _kernel_gradients(*grads):
             again = torch.is_grad_enabled()
             found = []
-            for x, w, g, (eps, repeat) in zip(xs, weights, grads, ctx.cfg):
-                with torch.enable_grad():
-                    y = x if w is None else rotate(rms_norm(x, w, eps), cos, sin)
-                    y = y.repeat_interleave(repeat, dim=2)
-                found += [torch.autograd.grad(y, x, g, create_graph=again)[0]
-                          if x.requires_grad else None, None]
+            for (x, w), g, heads, (eps, repeat) in zip(pairs, grads, ctx.heads, ctx.cfg):
+                dx = None
+                if w is None:
+                    dx = g.reshape(*g.shape[:2], heads, repeat, g.shape[3]).sum(3)
+                elif x.requires_grad:
+                    with torch.enable_grad():
+                        y = rotate(rms_norm(x, w, eps), cos, sin).repeat_interleave(repeat, dim=2)
+                    dx, = torch.autograd.grad(y, x, g, create_graph=again)
+                found += [dx, None]
             return (None, None, None, *found)
         grads = [g if g.stride(3) == 1 and not any(n % 8 for n in g.stride()[:3])
                  and g.data_ptr() % 16 == 0 else _aligned(g) for g in grads]
-        outs = [torch.empty_like(x) for x in xs]
-        _head_norm(cos, sin, ctx.cfg, xs, weights, grads, outs)
+        outs = [torch.empty((*g.shape[:2], heads, g.shape[3]), dtype=BF16, device=g.device)
+                for g, heads in zip(grads, ctx.heads)]
+        # where there is no norm to go back through, no row is read
+        xs = [dx if x is None else x for (x, _), dx in zip(pairs, outs)]
+        _head_norm(cos, sin, ctx.cfg, xs, [w for _, w in pairs], grads, outs)
         return (None, None, None, *(t for dx in outs for t in (dx, None)))
 
 
@@ -259,13 +274,17 @@ class RMSNorm(torch.nn.Module):
 
     def forward(self, value: torch.Tensor) -> torch.Tensor:
         if _row_kernel(value, self.weight):
+            if torch.is_grad_enabled() and value.requires_grad:
+                # the expression keeps a float32 copy, so its argument may
+                # change in place before the backward: keep a copy here too
+                return AddNormFn.apply(value, None, self.weight, None, nat.NORM_RMS, self.eps)[1]
             return NormFn.apply(value, self.weight, None, nat.NORM_RMS, self.eps)
         return rms_norm(value, self.weight, self.eps)
 
 
 def add_norm(norm: torch.nn.Module, value: torch.Tensor, update: torch.Tensor):
     """``t = value + update`` and ``norm(t)``: ``(t, norm(t))``, in one pass
-    where the kernels apply."""
+    where the kernels apply. The backward reads t: it must not change in place."""
 
     kind = {LayerNorm: nat.NORM_LAYER, RMSNorm: nat.NORM_RMS}.get(type(norm))
     if kind is not None and eager_calls() and _unhooked(norm, type(norm)):
@@ -285,7 +304,8 @@ def attention_heads(query_norm: torch.nn.Module, key_norm: torch.nn.Module, q: t
     """The operands of grouped-query attention from ``[B, S, H, D]`` projections:
     queries and keys through their norms, rotated by ``[1, S, D]`` float32
     angles and rounded to ``dtype``, key and value heads repeated to the
-    queries' count. One launch where the kernels apply."""
+    queries' count. One launch where the kernels apply; its backward reads q and
+    k, which must not change in place."""
 
     b, s, h, d = q.shape
     repeat = h // k.shape[2]

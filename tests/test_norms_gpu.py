@@ -258,6 +258,42 @@ def test_transforms_and_compilers_on_the_device():
 
 
 @pytest.mark.gpu
+def test_the_argument_of_an_rms_norm_may_change_before_the_backward():
+    """The expression saves a float32 copy of a bf16 row, so changing the row in
+    place after the call (x += ..., an RMSNorm's usual neighbour) is allowed.
+    The LayerNorm's expression saves its argument, where it is not."""
+
+    leaf = torch.randn(5, 64, device=DEV).to(BF16).requires_grad_(True)
+    dy = torch.randn(5, 64, device=DEV).to(BF16)
+    norm = _module("rms", 64)
+    got = []
+    for change in (False, True):
+        x = leaf * 1.0
+        y = norm(x)
+        assert "NormFn" in type(y.grad_fn).__name__
+        if change:
+            x.add_(1.0)
+        got.append((y.detach().clone(), *torch.autograd.grad(y, leaf, dy)))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    x = leaf * 1.0
+    y = norm(x)
+    (dx,) = torch.autograd.grad(y.float().square().sum(), x, create_graph=True)
+    assert torch.autograd.grad(dx.float().sum(), leaf)[0].shape == leaf.shape
+
+
+@pytest.mark.gpu
+def test_heads_that_are_only_repeated_are_not_kept():
+    q, k, v = (torch.randn(1, 3, n, 64, device=DEV).to(BF16).requires_grad_(True) for n in (4, 2, 2))
+    angle = torch.randn(1, 3, 32, device=DEV).repeat(1, 1, 2)
+    norm = _module("rms", 64)
+    outs = attention_heads(norm, norm, q, k, v, angle.cos(), angle.sin(), BF16)
+    kept = outs[2].grad_fn.saved_tensors
+    assert len(kept) == 6 and not any(t is v for t in kept)
+    (dv,) = torch.autograd.grad(outs[2], v, torch.ones_like(outs[2]), create_graph=True)
+    assert torch.equal(dv, torch.full_like(v, 2.0))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("create_graph", [False, True])
 def test_batched_gradients(create_graph):
     """Several gradients at once (is_grads_batched, vectorized Jacobians) have
