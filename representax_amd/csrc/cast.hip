@@ -14,13 +14,15 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kPerBlock = kThreads * 8;
 
-// Block b belongs to the tensor t with first[t] <= b < first[t + 1]; a thread
-// converts 8 consecutive elements.
+// Block b belongs to the tensor t with first[t] <= b < first[t + 1] (the last,
+// first[kCastMany], is the blocks' end); a thread converts 8 consecutive
+// elements.
 __global__ void __launch_bounds__(kThreads) k_cast_many(CastMany args) {
+  const int64_t block = block_of_grid();
+  if (block >= args.first[kCastMany]) return;
   int t = 0;
-  while (static_cast<int64_t>(blockIdx.x) >= args.first[t + 1]) ++t;
-  const int64_t i =
-      (blockIdx.x - args.first[t]) * kPerBlock + static_cast<int64_t>(threadIdx.x) * 8;
+  while (block >= args.first[t + 1]) ++t;
+  const int64_t i = (block - args.first[t]) * kPerBlock + static_cast<int64_t>(threadIdx.x) * 8;
   const int64_t n = args.count[t];
   const float* src = args.src[t];
   uint16_t* dst = args.dst[t];
@@ -39,11 +41,10 @@ __global__ void __launch_bounds__(kThreads) k_cast_many(CastMany args) {
 
 hipError_t launch_cast_many(CastMany args, int tensors, hipStream_t stream) {
   args.first[0] = 0;
-  for (int t = 0; t < tensors; ++t)
-    args.first[t + 1] = args.first[t] + ceil_div(args.count[t], kPerBlock);
+  for (int t = 0; t < kCastMany; ++t)
+    args.first[t + 1] = args.first[t] + (t < tensors ? ceil_div(args.count[t], kPerBlock) : 0);
   if (args.first[tensors] == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_cast_many, dim3(static_cast<unsigned>(args.first[tensors])),
-                     dim3(kThreads), 0, stream, args);
+  hipLaunchKernelGGL(k_cast_many, grid_of(args.first[tensors]), dim3(kThreads), 0, stream, args);
   return hipGetLastError();
 }
 

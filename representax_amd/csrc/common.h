@@ -114,6 +114,19 @@ constexpr int kErrInvalid = 1;
 constexpr int kErrHip = 2;
 constexpr int kErrDevice = 3;
 
-inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+__host__ __device__ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Grids of any number of workgroups. A launch holds fewer than 2^32 threads in
+// each dimension (2^22 workgroups of 1024), so workgroups past 2^21 continue in
+// rows of the second dimension; the last row can run past the end, where the
+// kernel returns.
+inline dim3 grid_of(int64_t blocks) {
+  const int64_t row = int64_t{1} << 21;
+  return blocks <= row ? dim3(static_cast<unsigned>(blocks))
+                       : dim3(static_cast<unsigned>(row), static_cast<unsigned>(ceil_div(blocks, row)));
+}
+__device__ __forceinline__ int64_t block_of_grid() {
+  return static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+}
 
 }  // namespace rpx

@@ -219,8 +219,10 @@ __global__ void __launch_bounds__(256 * G)
   const int wave = tid >> 6;
   float* const sa = lds + group * 4 * kBuf;  // two buffers each
   float* const sb = sa + 2 * kBuf;
-  const int64_t m0 = (blockIdx.x / tiles_n) * kTile;
-  const int64_t n0 = (blockIdx.x % tiles_n) * kTile;
+  const int64_t tile = block_of_grid();
+  if (tile >= ceil_div(M, kTile) * tiles_n) return;
+  const int64_t m0 = tile / tiles_n * kTile;
+  const int64_t n0 = tile % tiles_n * kTile;
   const int wm = 32 * (wave & 1);
   const int wn = 32 * (wave >> 1);
   f32x16_t acc;
@@ -310,8 +312,7 @@ hipError_t run_f32_groups(const F32Operand& a, const F32Operand& b, int64_t m, i
   static std::atomic<unsigned> lds_set{0};
   const hipError_t e = ensure_lds_limit(reinterpret_cast<const void*>(kern), kLds, lds_set);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(ceil_div(m, kTile) * ceil_div(n, kTile))),
-                     dim3(256 * G), kLds, stream, a, b, m, n, k, ceil_div(n, kTile), out);
+  hipLaunchKernelGGL(kern, grid_of(ceil_div(m, kTile) * ceil_div(n, kTile)), dim3(256 * G), kLds, stream, a, b, m, n, k, ceil_div(n, kTile), out);
   return hipGetLastError();
 }
 
@@ -367,8 +368,10 @@ __global__ void __launch_bounds__(64 * kThinWaves)
   __shared__ f32x4_t red[kThinWaves - 1][64];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int64_t m0 = (blockIdx.x / tiles_n) * 16;
-  const int64_t n0 = (blockIdx.x % tiles_n) * 16;
+  const int64_t tile = block_of_grid();
+  if (tile >= ceil_div(M, 16) * tiles_n) return;
+  const int64_t m0 = tile / tiles_n * 16;
+  const int64_t n0 = tile % tiles_n * 16;
   f32x4_t acc{0.0f, 0.0f, 0.0f, 0.0f};
   constexpr int U = 4;  // steps in flight
   for (int64_t k0 = wave * kThinK; k0 < K; k0 += U * kThinWaves * kThinK) {
@@ -452,8 +455,7 @@ hipError_t launch_generic_gemm(const void* a, int a_dtype, int64_t a_sm, int64_t
   // waves nothing to split.
   if (thin && k > 2 * kThinK) {
     auto run = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles)), dim3(64 * kThinWaves), 0, stream,
-                         oa, ob, m, n, k, tiles_n, out);
+      hipLaunchKernelGGL(kern, grid_of(tiles), dim3(64 * kThinWaves), 0, stream, oa, ob, m, n, k, tiles_n, out);
     };
     if (oa.kind == kAlongK && ob.kind == kAlongK)
       run(k_gemm_f32_thin<kAlongK, kAlongK>);

@@ -104,7 +104,7 @@ __global__ void __launch_bounds__(kThreads)
                const void* __restrict__ w, const void* __restrict__ b, int w_dtype, int64_t rows,
                int size, float eps, uint16_t* __restrict__ sum, uint16_t* __restrict__ y) {
   const int lane = threadIdx.x & (L - 1);
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * (kThreads / L) + threadIdx.x / L;
+  const int64_t row = block_of_grid() * (kThreads / L) + threadIdx.x / L;
   if (row >= rows) return;
   const int64_t base = row * size;
   float v[C][8];
@@ -182,7 +182,7 @@ __global__ void __launch_bounds__(kThreads)
                const uint16_t* __restrict__ t, const void* __restrict__ w, int w_dtype,
                int64_t rows, int size, float eps, uint16_t* __restrict__ dx) {
   const int lane = threadIdx.x & (L - 1);
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * (kThreads / L) + threadIdx.x / L;
+  const int64_t row = block_of_grid() * (kThreads / L) + threadIdx.x / L;
   if (row >= rows) return;
   const int64_t base = row * size;
   float v[C][8], g[C][8];
@@ -227,21 +227,23 @@ __global__ void __launch_bounds__(kThreads)
 // Heads of D = 8 * L elements, one per L lanes: lane l holds the elements
 // 8 l .. 8 l + 7, so the rotation's other half is lane l ^ (L / 2). The parts
 // (queries, keys and the values that only repeat) share a launch: blocks
-// [first[p], first[p + 1]) are part p's. x [tokens, heads, D] dense; y [tokens,
+// [first[p], first[p + 1]) are part p's, and first[kHeadParts] is their end. x [tokens, heads, D] dense; y [tokens,
 // heads * repeat, D] dense, head h written `repeat` times.
-__device__ __forceinline__ int head_part(const HeadNormArgs& a) {
+__device__ __forceinline__ int head_part(const HeadNormArgs& a, int64_t block) {
   int p = 0;
-  while (static_cast<int64_t>(blockIdx.x) >= a.first[p + 1]) ++p;
+  while (block >= a.first[p + 1]) ++p;
   return p;
 }
 
 template <int L>
 __global__ void __launch_bounds__(kThreads) k_head_norm_fwd(HeadNormArgs a) {
   constexpr int kD = 8 * L;
-  const int p = head_part(a);
+  const int64_t block = block_of_grid();
+  if (block >= a.first[kHeadParts]) return;
+  const int p = head_part(a, block);
   const HeadPart& part = a.part[p];
   const int lane = threadIdx.x & (L - 1);
-  const int64_t row = (blockIdx.x - a.first[p]) * (kThreads / L) + threadIdx.x / L;
+  const int64_t row = (block - a.first[p]) * (kThreads / L) + threadIdx.x / L;
   if (row >= a.tokens * part.heads) return;
   const int64_t token = row / part.heads;
   const int e = 8 * lane;
@@ -271,10 +273,12 @@ __global__ void __launch_bounds__(kThreads) k_head_norm_fwd(HeadNormArgs a) {
 template <int L>
 __global__ void __launch_bounds__(kThreads) k_head_norm_bwd(HeadNormArgs a) {
   constexpr int kD = 8 * L;
-  const int p = head_part(a);
+  const int64_t block = block_of_grid();
+  if (block >= a.first[kHeadParts]) return;
+  const int p = head_part(a, block);
   const HeadPart& part = a.part[p];
   const int lane = threadIdx.x & (L - 1);
-  const int64_t row = (blockIdx.x - a.first[p]) * (kThreads / L) + threadIdx.x / L;
+  const int64_t row = (block - a.first[p]) * (kThreads / L) + threadIdx.x / L;
   if (row >= a.tokens * part.heads) return;
   const int64_t token = row / part.heads;
   const int64_t s = token % a.sequence;
@@ -317,16 +321,14 @@ __global__ void __launch_bounds__(kThreads) k_head_norm_bwd(HeadNormArgs a) {
 template <int KIND, bool ADD, int L, int C>
 void norm_fwd(const NormArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL((k_norm_fwd<KIND, ADD, L, C>),
-                     dim3(static_cast<unsigned>(ceil_div(a.rows, kThreads / L))), dim3(kThreads),
-                     0, stream, a.x, a.residual, a.weight, a.bias, a.weight_dtype, a.rows, a.size,
+                     grid_of(ceil_div(a.rows, kThreads / L)), dim3(kThreads), 0, stream, a.x, a.residual, a.weight, a.bias, a.weight_dtype, a.rows, a.size,
                      a.eps, a.sum, a.y);
 }
 
 template <int KIND, bool ADD, int L, int C>
 void norm_bwd(const NormArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL((k_norm_bwd<KIND, ADD, L, C>),
-                     dim3(static_cast<unsigned>(ceil_div(a.rows, kThreads / L))), dim3(kThreads),
-                     0, stream, a.x, a.residual, a.sum, a.weight, a.weight_dtype, a.rows, a.size,
+                     grid_of(ceil_div(a.rows, kThreads / L)), dim3(kThreads), 0, stream, a.x, a.residual, a.sum, a.weight, a.weight_dtype, a.rows, a.size,
                      a.eps, a.y);
 }
 
@@ -358,13 +360,13 @@ hipError_t launch_norm(const NormArgs& a, int kind, bool backward, hipStream_t s
 hipError_t launch_head_norm(HeadNormArgs a, int parts, bool backward, hipStream_t stream) {
   const int lanes = a.head_dim / 8;
   a.first[0] = 0;
-  for (int p = 0; p < parts; ++p)
-    a.first[p + 1] = a.first[p] + ceil_div(a.tokens * a.part[p].heads, kThreads / lanes);
+  for (int p = 0; p < kHeadParts; ++p)
+    a.first[p + 1] =
+        a.first[p] + (p < parts ? ceil_div(a.tokens * a.part[p].heads, kThreads / lanes) : 0);
   if (a.first[parts] == 0) return hipSuccess;
   const auto kernel = a.head_dim == 128 ? (backward ? k_head_norm_bwd<16> : k_head_norm_fwd<16>)
                                         : (backward ? k_head_norm_bwd<8> : k_head_norm_fwd<8>);
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(a.first[parts])), dim3(kThreads), 0,
-                     stream, a);
+  hipLaunchKernelGGL(kernel, grid_of(a.first[parts]), dim3(kThreads), 0, stream, a);
   return hipGetLastError();
 }
 

@@ -81,3 +81,25 @@ def test_float32_linear_keeps_infinities_nan_and_tiny_values():
     assert torch.equal(y[rest], x[rest] @ w.t())
     small, _ = ops.int4lora_forward(x[65:] * 1e-4, packed, scales, zero_a, zero_b, scaling=1.0)
     assert torch.equal(small[1, 63], (x[66, 63] * 1e-4) * w[63, 63]) and small[1, 63] != 0
+
+
+def test_more_tiles_than_one_grid_dimension():
+    """2^26 rows and three more are more thin tiles than a launch holds in one
+    dimension: the rows around the limits equal a small call's, bit for bit."""
+
+    m, k, n, r = (1 << 26) + 3, 40, 2, 1
+    g = torch.Generator(device="cuda").manual_seed(3)
+    base = torch.randn((1 << 12, k), generator=g, device="cuda")
+    packed, scales = ops.int4_pack(torch.randn((n, k), generator=g, device="cuda"))
+    a, b = (torch.randn(s, generator=g, device="cuda") for s in ((r, k), (n, r)))
+    want, h_want = ops.int4lora_forward(base, packed, scales, a, b, scaling=1.5)
+    x = torch.empty((m, k), device="cuda")
+    x[:1 << 26].view(1 << 14, 1 << 12, k).copy_(base.expand(1 << 14, 1 << 12, k))
+    x[1 << 26:] = base[:3]
+    y, h = ops.int4lora_forward(x, packed, scales, a, b, scaling=1.5)
+    for got, part in ((y, want), (h, h_want)):
+        for at in (0, 1 << 25, (1 << 26) - (1 << 12)):  # row 0, the second grid row, the last
+            assert torch.equal(got[at:at + (1 << 12)], part)
+        assert torch.equal(got[1 << 26:], part[:3])
+    del x, y, h, got
+    torch.cuda.empty_cache()

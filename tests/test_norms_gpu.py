@@ -258,6 +258,59 @@ def test_transforms_and_compilers_on_the_device():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["layer", "rms"])
+def test_more_rows_than_one_grid_dimension(kind):
+    """2^28 rows of 8 elements are 2^32 lanes, one more than a launch holds in a
+    dimension: the rows on both sides of the limit equal the same rows' norms
+    in a small call, forward and backward."""
+
+    rows = (1 << 28) + 5
+    g = torch.Generator(device=DEV).manual_seed(1)
+    base, grad = (torch.randn(1 << 14, 8, generator=g, device=DEV).to(BF16) for _ in range(2))
+    x, dy = (t.repeat(1 << 14, 1)[:rows] for t in (base, grad))
+    x = torch.cat((x, base[:5]))[:rows].requires_grad_(True)
+    dy = torch.cat((dy, grad[:5]))[:rows]
+    norm = _module(kind, 8)
+    y = norm(x)
+    assert "NormFn" in type(y.grad_fn).__name__
+    (dx,) = torch.autograd.grad(y, x, dy)
+    small = base.clone().requires_grad_(True)
+    want = norm(small)
+    (dwant,) = torch.autograd.grad(want, small, grad)
+    for got, part in ((y.detach(), want.detach()), (dx, dwant)):
+        for at in (0, 1 << 25, (1 << 28) - (1 << 14)):  # row 0, the second grid row, the last
+            assert torch.equal(got[at:at + (1 << 14)], part)
+        assert torch.equal(got[1 << 28:], part[:5])
+    del x, y, dx, dy, got
+    torch.cuda.empty_cache()
+
+
+@pytest.mark.gpu
+def test_more_heads_than_one_grid_row():
+    """2^21 workgroups of 32 heads and a few more: the second row of the grid."""
+
+    s, h, d = (1 << 19) + 8, 128, 64
+    g = torch.Generator(device=DEV).manual_seed(2)
+    q = torch.randn(1, 64, h, d, generator=g, device=DEV).to(BF16)
+    k, v = (torch.randn(1, 64, 1, d, generator=g, device=DEV).to(BF16) for _ in range(2))
+    angle = torch.randn(1, 64, d // 2, generator=g, device=DEV).repeat(1, 1, 2)
+    norm = _module("rms", d)
+    want = attention_heads(norm, norm, q, k, v, angle.cos(), angle.sin(), BF16)
+
+    def many(t):
+        return t.repeat(1, -(-s // 64), *([1] * (t.dim() - 2)))[:, :s].contiguous()
+
+    got = attention_heads(norm, norm, many(q), many(k), many(v), many(angle.cos()),
+                          many(angle.sin()), BF16)
+    for a, b in zip(got, want):
+        for at in (0, 1 << 18, s - 8 - 64):
+            assert torch.equal(a[:, at:at + 64], b)
+        assert torch.equal(a[:, s - 8:], b[:, :8])
+    del got, a
+    torch.cuda.empty_cache()
+
+
+@pytest.mark.gpu
 def test_the_argument_of_an_rms_norm_may_change_before_the_backward():
     """The expression saves a float32 copy of a bf16 row, so changing the row in
     place after the call (x += ..., an RMSNorm's usual neighbour) is allowed.
