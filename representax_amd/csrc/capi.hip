@@ -128,11 +128,25 @@ void plan_forward(A& a, bool fast, bool skinny, int64_t m, int64_t n, int64_t k,
   a.template take<float>(m * rank);
 }
 
+// The LoRA term of a forward on the MFMA path, without its pointers.
+LowRankEpilogue forward_epilogue(int64_t rank, int act) {
+  LowRankEpilogue epi;
+  epi.rows_sn = rank;
+  epi.rows_sj = 1;
+  epi.cols_sm = rank;
+  epi.cols_sj = 1;
+  epi.rank = rank;
+  epi.act = act;
+  return epi;
+}
+
 // The persistent wide GEMM's tile id for a forward on the MFMA path (0: the
-// fused dequantizing GEMM). It reads a bf16 copy of W_b [n, k] from the
-// workspace; a call whose workspace has no room for that copy takes the fused
-// GEMM, which needs none.
-int forward_wide_tile(int64_t m, int64_t n, int64_t k, int act) {
+// fused dequantizing GEMM, which sizes and ranks without a wide kernel always
+// take). It reads a bf16 copy of W_b [n, k] from the workspace; a call whose
+// workspace has no room for that copy takes the fused GEMM, which needs none.
+int forward_wide_tile(int64_t m, int64_t n, int64_t k, int64_t rank, int act) {
+  if (!wide_gemm_ok(nullptr, k, nullptr, k, m, n, k, nullptr, n, forward_epilogue(rank, act)))
+    return 0;
   return wide_plan(m, n, k, tune(kTuneInt4Tile), act, true);
 }
 
@@ -427,7 +441,7 @@ size_t rpx_int4lora_forward_workspace(int64_t m, int64_t n, int64_t k, int64_t g
   const bool fast = lora_fast_shape(dtype, k, ng, g, rank);
   const bool skinny = lora_skinny(dtype, m, n, k, ng, g, rank);
   plan_forward(s, fast, skinny, m, n, k, rank);
-  if (fast && !skinny && m > 0 && n > 0 && forward_wide_tile(m, n, k, kActNone) != 0)
+  if (fast && !skinny && m > 0 && n > 0 && forward_wide_tile(m, n, k, rank, kActNone) != 0)
     s.take<uint16_t>(n * k);  // W_b
   return s.used;
 }
@@ -513,20 +527,14 @@ int int4lora_forward_impl(const void* x, int dtype, int64_t m, int64_t k, const 
       RPX_HIP(launch_rank_nt(xb, k, static_cast<const uint16_t*>(lora_a), k, m, rank, k, false,
                              1.0f, hb, rank, st),
               "int4lora_forward: adapter down-projection");
-    LowRankEpilogue epi;
+    LowRankEpilogue epi = forward_epilogue(rank, act.mode);
     epi.rows = static_cast<const uint16_t*>(lora_b);
-    epi.rows_sn = rank;
-    epi.rows_sj = 1;
     epi.cols = hb;
-    epi.cols_sm = rank;
-    epi.cols_sj = 1;
-    epi.rank = rank;
     epi.scale = c;
     epi.bias = bias_bits;
-    epi.act = act.mode;
     epi.aux = act.aux;
     epi.pre_out = act.pre_out;
-    const int wide = forward_wide_tile(m, n, k, act.mode);
+    const int wide = forward_wide_tile(m, n, k, rank, act.mode);
     if (wide != 0) {
       uint16_t* wb = arena.take<uint16_t>(n * k);
       if (!arena.overflow && wide_gemm_ok(xb, k, wb, k, m, n, k, static_cast<uint16_t*>(y), n, epi)) {

@@ -591,13 +591,15 @@ bool wide_gemm_ok(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb
       reinterpret_cast<uintptr_t>(epi.out2) | reinterpret_cast<uintptr_t>(epi.rows) |
       reinterpret_cast<uintptr_t>(epi.cols);
   // 32-bit row offsets of the operands; 16-byte pieces everywhere; a LoRA
-  // term of rank 16 or 32 with unit stride (more fragments would spill: 48
-  // and 64 stay with the smaller tiles)
+  // term of rank 16 or 32 with unit stride: two 16-rank blocks are what the
+  // epilogue has registers for (48 and 64 would spill), and its loads read whole
+  // blocks, so other ranks, also below 16, stay with k_gemm_nt, which pads them
   const int64_t lim = int64_t{1} << 32;
   return m > 0 && n > 0 && k > 0 && k % kBK == 0 && lda % 8 == 0 && ldb % 8 == 0 && n % 8 == 0 &&
          ldc % 8 == 0 && (ptrs & 15) == 0 && m * lda * 2 < lim && n * ldb * 2 < lim &&
          m < (int64_t{1} << 31) - 256 && n < (int64_t{1} << 31) - 256 &&
-         ceil_div(m, 256) * ceil_div(n, 192) < (int64_t{1} << 30) && (epi.rank == 16 || epi.rank == 32 || (epi.rank == 0 && epi.act == kActNone)) &&
+         ceil_div(m, 256) * ceil_div(n, 192) < (int64_t{1} << 30) &&
+         (epi.rank == 16 || epi.rank == 32 || (epi.rank == 0 && epi.act == kActNone)) &&
          (epi.rank == 0 || (epi.rows_sj == 1 && epi.cols_sj == 1 && epi.rows_sn % 8 == 0 &&
                             epi.cols_sm % 8 == 0 && m * epi.cols_sm * 2 < lim &&
                             n * epi.rows_sn * 2 < lim)) &&

@@ -46,6 +46,18 @@ def test_workspace_queries():
     assert lib.rpx_fp8_linear_backward_workspace(8192, 3072, 768) >= 8192 * 3072 + 768 * 3072 + 8192 * 768
 
 
+@pytest.mark.parametrize("m,n,k,rank,copy", [
+    (16384, 6144, 2048, 32, True), (16384, 6144, 2048, 16, True), (32768, 3072, 768, 16, True),
+    (16384, 6144, 2048, 8, False), (16384, 6144, 2048, 24, False), (16384, 6144, 2048, 64, False),
+    (1 << 20, 2048, 2048, 32, False), (333, 6144, 2048, 32, False)])
+def test_forward_workspace_holds_the_weight_copy_only_where_it_is_read(m, n, k, rank, copy):
+    """The bf16 weight copy of the large forwards: not for ranks or sizes (rows
+    beyond 32-bit offsets) that the GEMM over it does not take."""
+
+    need = nat.load().rpx_int4lora_forward_workspace(m, n, k, 64, rank, nat.DTYPE_BF16)
+    assert need >= 2 * n * k if copy else need == 0
+
+
 def test_invalid_arguments_are_rejected_before_any_launch():
     p = ctypes.c_void_p(16)  # never dereferenced: validation fails first
     with pytest.raises(ValueError, match="group_size"):
