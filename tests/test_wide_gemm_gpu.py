@@ -13,6 +13,7 @@ import pytest
 import torch
 
 from representax_amd import ops
+from tests.helpers import kernel_names
 
 pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
@@ -99,3 +100,67 @@ def test_without_workspace_takes_the_fused_gemm():
                  p["b"].data_ptr(), r, 2.0, y.data_ptr(), h.data_ptr(), None, 0,
                  torch.cuda.current_stream().cuda_stream)
     assert torch.equal(y, want) and torch.equal(h, h_want)
+
+
+@pytest.mark.parametrize("r,wide", [(16, True), (32, True), (24, False)])
+def test_automatic_choice(r, wide):
+    """Without a forced tile: the large products of rank 16 and 32 run the wide
+    kernel, forward and input gradient, and another rank runs none of it, with
+    the bits of the forced small tile either way."""
+
+    m, k, n = 16384, 768, 3072
+    p = _operands(m, k, n, r, 64, True)
+
+    def forward():
+        return ops.int4lora_forward(p["x"], p["packed"], p["scales"], p["a"], p["b"], scaling=1.7,
+                                    group_size=64, bias_bits=p["bias"])
+
+    (y, h), names = kernel_names(forward)
+    assert any("k_gemm_wide" in name for name in names) == wide
+    with ops.tuning(int4_tile=3):
+        want, _ = forward()
+    assert torch.equal(y, want)
+
+    def backward():
+        return ops.int4lora_backward(p["gy"], p["x"], p["packed"], p["scales"], p["a"], p["b"], h,
+                                     scaling=1.7, group_size=64)
+
+    got, names = kernel_names(backward)
+    assert any("k_gemm_wide" in name for name in names) == wide
+    with ops.tuning(bf16_tile=6):
+        want = backward()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+# more tiles than the 256 workgroups, so that the load pipeline runs on into a
+# second tile, over reductions of two and three 64-deep slices (the stages'
+# parity carries over), ragged rows and columns: (m, reduction, forward columns,
+# input gradient's columns, rank)
+SECOND_TILE = [(257 * 256 + 65, 128, 200, 192, 16), (257 * 256 + 65, 192, 200, 192, 32),
+               (130 * 256 + 3, 192, 584, 576, 16)]
+
+
+@pytest.mark.parametrize("m,k,n,columns,r", SECOND_TILE)
+def test_second_tile_of_a_workgroup(m, k, n, columns, r):
+    p = _operands(m, k, n, r, 64, True)
+    back = _operands(m, columns, k, r, None, False)  # its input gradient reduces over k
+
+    def forward(tile):
+        with ops.tuning(int4_tile=tile):
+            return ops.int4lora_forward_act(p["x"], p["packed"], p["scales"], p["a"], p["b"],
+                                            activation="gelu", scaling=1.7, group_size=64,
+                                            bias_bits=p["bias"])
+
+    def backward(tile):
+        with ops.tuning(bf16_tile=tile):
+            return ops.int4lora_backward_act(back["gy"], back["x"], back["packed"], back["scales"],
+                                             back["a"], back["b"], back["gy"][:, :r].contiguous(),
+                                             activation="gelu", z=back["zx"], scaling=2.0)
+
+    for run, small in ((forward, 3), (backward, 6)):
+        want = run(small)
+        for tile in WIDE:
+            got, names = kernel_names(lambda: run(tile))
+            assert any("k_gemm_wide" in name for name in names), (run.__name__, tile)
+            for w, g in zip(want, got):
+                assert w is None or torch.equal(w, g), (run.__name__, tile)
