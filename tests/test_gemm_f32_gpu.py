@@ -4,8 +4,10 @@ against float64 with the bound of a float32 sum.
 A sum of n float32 products is within n * 2^-24 * sum |a||b| of the exact one
 whatever its order (first order in 2^-24; 2^-23 below leaves room for the
 higher ones), and each later product adds its own term. The shapes sit around
-the kernels' edges: 16 x 16 and 64 x 64 outputs, K blocks of 32 and thin steps
-of 128, odd K, group scales of 2 (one element at a time) and of 64.
+the kernels' edges: 16 x 16 and 64 x 64 outputs, K blocks of 32 (taken in turn
+by four groups of waves from K = 256 on: last rounds in which some groups have a
+part of a block or none, forward and input gradient) and thin steps of 256, odd
+K, group scales of 2 (one element at a time), 4 and 64.
 """
 
 from __future__ import annotations
@@ -30,7 +32,8 @@ def _exact_weight(packed, scales, k):
 
 # (m, k, n, r, group)
 SHAPES = [(1, 33, 5, 1, None), (63, 64, 65, 3, 2), (65, 100, 129, 16, 4), (64, 31, 64, 17, None),
-          (200, 768, 192, 65, 64), (129, 1, 70, 1, None), (3000, 96, 48, 2, 32)]
+          (200, 768, 192, 65, 64), (129, 1, 70, 1, None), (3000, 96, 48, 2, 32),
+          (130, 300, 330, 3, 4), (70, 420, 290, 17, None), (67, 261, 259, 1, None)]
 
 
 @pytest.mark.parametrize("m,k,n,r,group", SHAPES)
@@ -68,18 +71,22 @@ def test_float32_linear_keeps_infinities_nan_and_tiny_values():
     products in the subnormal range are kept (no operand is split)."""
 
     m, k, n, r = 70, 64, 80, 2
+    inf = float("inf")
     packed, scales = ops.int4_pack(torch.eye(n, k, device="cuda") * 7.0)
     x = torch.zeros((m, k), device="cuda")
-    x[3, 5], x[4, 6], x[66, 63] = float("inf"), float("nan"), 1e-38
-    zero_a, zero_b = torch.zeros((r, k), device="cuda"), torch.zeros((n, r), device="cuda")
+    x[3, 5], x[4, 6], x[66, 63] = inf, float("nan"), 1e-38
+    # the adapter passes on column 5 alone, so that its infinity stays one
+    a, b = torch.zeros((r, k), device="cuda"), torch.ones((n, r), device="cuda")
+    a[:, 5] = 1.0
     w = ops.int4_dequant(packed, scales, k).float()
-    y, _ = ops.int4lora_forward(x, packed, scales, zero_a, zero_b, scaling=1.0)
-    # rows 3 and 4 are NaN wherever inf or nan meets a zero weight
-    assert torch.isnan(y[4]).all()
-    assert y[3, 5] == float("inf") or torch.isnan(y[3, 5])
+    y, h = ops.int4lora_forward(x, packed, scales, a, b, scaling=1.0)
+    # infinity times the weight's zeros is NaN; column 5 has none
+    assert torch.isnan(y[4]).all() and torch.isnan(h[4]).all() and (h[3] == inf).all()
+    others = [j for j in range(n) if j != 5]
+    assert y[3, 5] == inf and torch.isnan(y[3, others]).all()
     rest = [i for i in range(m) if i not in (3, 4)]
     assert torch.equal(y[rest], x[rest] @ w.t())
-    small, _ = ops.int4lora_forward(x[65:] * 1e-4, packed, scales, zero_a, zero_b, scaling=1.0)
+    small, _ = ops.int4lora_forward(x[65:] * 1e-4, packed, scales, a, b, scaling=1.0)
     assert torch.equal(small[1, 63], (x[66, 63] * 1e-4) * w[63, 63]) and small[1, 63] != 0
 
 
