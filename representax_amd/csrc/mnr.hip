@@ -3,8 +3,9 @@
 // query's log-sum-exp, the mean over queries, and the gradient of all of it
 // (src/representax/tasks/retrieval/mnr.py:48-52 `_normalize`, :132-158
 // `_direction_row_terms` with query i's positive = document i and unit
-// weights, :338-341 the forward loss). Four launches replace the ~30 small
-// elementwise, reduction and matmul kernels of the unfused objective.
+// weights, :338-341 the forward loss). Five launches (four forward, one
+// backward) replace the ~30 small elementwise, reduction and matmul kernels of
+// the unfused objective.
 //
 // Every sum runs in a fixed order (per-thread strided partials, then a
 // shuffle tree, then the waves in order; MFMA chains, then the waves in

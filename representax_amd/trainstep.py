@@ -526,8 +526,9 @@ class MNRTrainStep:
             loss = mnr_loss(emb[:b], emb[b:], self.scale)
         loss.backward()
         grad = self.flat.grad
-        # bf16 view gradients -> the masters' float32 gradient, one kernel (a
-        # view that took no part in the loss has gradient zero)
+        # bf16 view gradients -> the masters' float32 gradient (the dtypes
+        # differ, so torch.cat copies one view at a time, a launch of 4 us
+        # each; a view that took no part in the loss has gradient zero)
         torch.cat([(v.grad if v.grad is not None else torch.zeros_like(v)).reshape(-1)
                    for v in self.view_list], out=grad)
         norm = torch.linalg.vector_norm(grad, dtype=torch.float32)
