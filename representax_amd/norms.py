@@ -66,17 +66,20 @@ def _frozen(size: int, device, *weights: torch.Tensor) -> bool:
 
     grad = torch.is_grad_enabled()
     return all(plain_tensor(w) and w.device == device and w.shape == (size,)
-               and w.dtype in (F32, BF16) and w.dtype == weights[0].dtype and _dense(w) and not (grad and w.requires_grad)
-               for w in weights)
+               and w.dtype in (F32, BF16) and w.dtype == weights[0].dtype and _dense(w)
+               and not (grad and w.requires_grad) for w in weights)
+
+
+def _rows_fit(value: torch.Tensor, *weights: torch.Tensor) -> bool:
+    size = value.shape[-1] if value.dim() else 0
+    return (plain_tensor(value) and value.dtype == BF16 and 8 <= size <= _MAX_SIZE
+            and size % 8 == 0 and 0 < value.numel() and value.numel() // size <= 1 << 31
+            and _dense(value) and _frozen(size, value.device, *weights)
+            and not torch.is_autocast_enabled("cuda"))
 
 
 def _row_kernel(value: torch.Tensor, *weights: torch.Tensor) -> bool:
-    if not eager_calls():
-        return False
-    size = value.shape[-1] if value.dim() else 0
-    return (plain_tensor(value) and value.dtype == BF16 and 8 <= size <= _MAX_SIZE
-            and size % 8 == 0 and 0 < value.numel() and value.numel() // size <= 1 << 31 and _dense(value)
-            and _frozen(size, value.device, *weights) and not torch.is_autocast_enabled("cuda"))
+    return eager_calls() and _rows_fit(value, *weights)
 
 
 def _unhooked(module: torch.nn.Module, cls: type) -> bool:
@@ -290,7 +293,7 @@ def add_norm(norm: torch.nn.Module, value: torch.Tensor, update: torch.Tensor):
     if kind is not None and eager_calls() and _unhooked(norm, type(norm)):
         bias = norm.bias if kind == nat.NORM_LAYER else None
         weights = (norm.weight,) if bias is None else (norm.weight, bias)
-        if (_row_kernel(value, *weights) and plain_tensor(update) and update.dtype == BF16
+        if (_rows_fit(value, *weights) and plain_tensor(update) and update.dtype == BF16
                 and update.shape == value.shape and update.device == value.device
                 and _dense(update)):
             return AddNormFn.apply(value, update, norm.weight, bias, kind, norm.eps)
@@ -313,7 +316,7 @@ def attention_heads(query_norm: torch.nn.Module, key_norm: torch.nn.Module, q: t
             and d in (64, 128)
             and dtype == BF16 and h <= 65536 and repeat * k.shape[2] == h
             and k.shape == v.shape == (b, s, k.shape[2], d)  # the launch reads b * s tokens of each
-            and _row_kernel(q, query_norm.weight) and _row_kernel(k, key_norm.weight)
+            and _rows_fit(q, query_norm.weight) and _rows_fit(k, key_norm.weight)
             and plain_tensor(v) and v.dtype == BF16 and _dense(v)
             and k.device == q.device == v.device
             and all(plain_tensor(t) and t.dtype == F32 and t.device == q.device

@@ -718,10 +718,10 @@ def cast_many(tensors, dtype: torch.dtype) -> list[torch.Tensor]:
     dense tensors of one device (no autograd)."""
 
     device = tensors[0].device
-    if not (dtype == BF16 and 1 < len(tensors) <= CAST_MANY and eager_calls()
-            and all(t.dtype == F32 and plain_tensor(t) and t.device == device
-                    and t.is_contiguous() and t.numel() and t.data_ptr() % 16 == 0
-                    for t in tensors)):
+    if not (dtype == BF16 and 1 < len(tensors) <= CAST_MANY
+            and all(t.dtype == F32 for t in tensors) and eager_calls()
+            and all(plain_tensor(t) and t.device == device and t.is_contiguous() and t.numel()
+                    and t.data_ptr() % 16 == 0 for t in tensors)):
         return [t.to(dtype) for t in tensors]
     out = [torch.empty_like(t, dtype=BF16) for t in tensors]
     count = len(tensors)

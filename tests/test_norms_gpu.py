@@ -178,7 +178,7 @@ def test_attention_heads_launches_only_over_matching_tokens(monkeypatch, kv, rou
 
     taken = []
     monkeypatch.setattr(norms, "plain_tensor", lambda t: True)
-    monkeypatch.setattr(norms, "_row_kernel", lambda *a: True)
+    monkeypatch.setattr(norms, "_rows_fit", lambda *a: True)
     monkeypatch.setattr(RMSNorm, "forward", lambda m, t: norms.rms_norm(t, m.weight, m.eps))
     monkeypatch.setattr(norms.HeadNormFn, "apply", lambda *a: taken.append(a) or (q, k, v))
     q, k, v = (torch.randn(s).to(BF16) for s in ((2, 5, 4, 64), kv, kv))
