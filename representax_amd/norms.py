@@ -18,7 +18,7 @@ import torch.nn.functional as F
 
 from . import _native as nat
 from .ops import (BF16, F32, _aligned, _dtype_code, _on_device, _ptr, _stream, eager_calls,
-                  plain_tensor)
+                  on_current_device, plain_tensor)
 
 _MAX_SIZE = 4096  # elements of a row that the kernels keep in registers
 
@@ -72,8 +72,9 @@ def _frozen(size: int, device, *weights: torch.Tensor) -> bool:
 
 def _rows_fit(value: torch.Tensor, *weights: torch.Tensor) -> bool:
     size = value.shape[-1] if value.dim() else 0
-    return (plain_tensor(value) and value.dtype == BF16 and 8 <= size <= _MAX_SIZE
-            and size % 8 == 0 and 0 < value.numel() and value.numel() // size <= 1 << 31
+    return (plain_tensor(value) and on_current_device(value) and value.dtype == BF16
+            and 8 <= size <= _MAX_SIZE and size % 8 == 0
+            and 0 < value.numel() and value.numel() // size <= 1 << 31
             and _dense(value) and _frozen(size, value.device, *weights)
             and not torch.is_autocast_enabled("cuda"))
 

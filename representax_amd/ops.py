@@ -11,6 +11,7 @@ import ctypes
 import math
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _native as nat
 
@@ -691,13 +692,29 @@ def int4lora_backward_act(grad, x2d, packed, scale_bits, lora_a_c, lora_b_c, h, 
 CAST_MANY = 16  # tensors of one launch
 
 
-def plain_tensor(t: torch.Tensor) -> bool:
-    """An ordinary device tensor: no subclass, no function-transform wrapper,
-    no batched gradient (those have no storage of their own)."""
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+_has_storage = torch._C._has_storage
 
-    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
-            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-            and torch._C._has_storage(t))
+
+def plain_tensor(t: torch.Tensor) -> bool:
+    """An ordinary device tensor: no subclass, no function-transform wrapper or
+    batched gradient (those have no storage of their own)."""
+
+    return type(t) in _TENSORS and t.is_cuda and _has_storage(t)
+
+
+def on_current_device(t: torch.Tensor) -> bool:
+    """The device tensor is where a launch goes: torch's operations follow their
+    tensors, a launch goes to the current device."""
+
+    return t.get_device() == torch._C._cuda_getDevice()
+
+
+_is_compiling = torch.compiler.is_compiling
+_tracing_state = torch._C._get_tracing_state
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+_transforms_active = torch._C._are_functorch_transforms_active
 
 
 def eager_calls() -> bool:
@@ -707,10 +724,8 @@ def eager_calls() -> bool:
     function transform an autograd function is refused also where its tensors
     are only closed over."""
 
-    return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
-                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-                or torch._C._are_functorch_transforms_active()
-                or torch.autograd.forward_ad._current_level >= 0)
+    return not (_is_compiling() or _tracing_state() is not None or _dispatch_modes()
+                or _function_modes() or _transforms_active() or forward_ad._current_level >= 0)
 
 
 def cast_many(tensors, dtype: torch.dtype) -> list[torch.Tensor]:
@@ -721,7 +736,8 @@ def cast_many(tensors, dtype: torch.dtype) -> list[torch.Tensor]:
     if not (dtype == BF16 and 1 < len(tensors) <= CAST_MANY
             and all(t.dtype == F32 for t in tensors) and eager_calls()
             and all(plain_tensor(t) and t.device == device and t.is_contiguous() and t.numel()
-                    and t.data_ptr() % 16 == 0 for t in tensors)):
+                    and t.data_ptr() % 16 == 0 for t in tensors)
+            and on_current_device(tensors[0])):
         return [t.to(dtype) for t in tensors]
     out = [torch.empty_like(t, dtype=BF16) for t in tensors]
     count = len(tensors)

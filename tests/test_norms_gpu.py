@@ -202,11 +202,10 @@ def _cpu_routes(monkeypatch):
     """The routes' conditions on CPU tensors: everything but their device."""
 
     def plain(t):
-        return (type(t) in (torch.Tensor, torch.nn.Parameter)
-                and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-                and torch._C._has_storage(t))
+        return type(t) in (torch.Tensor, torch.nn.Parameter) and torch._C._has_storage(t)
 
     monkeypatch.setattr(norms, "plain_tensor", plain)
+    monkeypatch.setattr(norms, "on_current_device", lambda t: True)
 
 
 def test_transforms_and_compilers_keep_the_expressions(monkeypatch):
@@ -332,6 +331,27 @@ def test_the_argument_of_an_rms_norm_may_change_before_the_backward():
     y = norm(x)
     (dx,) = torch.autograd.grad(y.float().square().sum(), x, create_graph=True)
     assert torch.autograd.grad(dx.float().sum(), leaf)[0].shape == leaf.shape
+
+
+@pytest.mark.gpu
+def test_tensors_of_another_device_than_the_current_one(monkeypatch):
+    """A launch goes to the current device; torch's operations go to their
+    tensors' device. Where the two differ the expressions run."""
+
+    x, r = (torch.randn(4, 64, device=DEV).to(BF16) for _ in range(2))
+    norm, masters = _module("rms", 64), [torch.randn(8, 8, device=DEV) for _ in range(2)]
+    want = norms.rms_norm(x + r, norm.weight, norm.eps)
+    assert norms._row_kernel(x, norm.weight)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 1)
+    assert not norms._row_kernel(x, norm.weight)
+
+    def no_launch(*args):
+        raise AssertionError(args[0])
+
+    monkeypatch.setattr(norms.nat, "call", no_launch)
+    assert torch.equal(add_norm(norm, x, r)[1], want) and torch.equal(norm(x + r), want)
+    for t, got in zip(masters, ops.cast_many(masters, BF16)):
+        assert torch.equal(got, t.to(BF16))
 
 
 @pytest.mark.gpu
